@@ -225,17 +225,57 @@ __device__ __forceinline__ void gather_tile_sums(const TileParts<R> &tp, int i, 
             }
 }
 
+// The sample of a point tool nearest to each node that asks (`need`; the
+// whole wave calls): among the samples at d2 < rc2 and > 1e-20 the one of
+// least d2, the first of equal ones (MPMWorkpieceSolver.cu:157-172), -1 for
+// none.  The tool box holds a few nodes of a wave, so a loop per node over all
+// samples left most lanes idle behind the few that ran it (845 samples of a
+// rake face over 131 thousand particles: 105 us of grid update): the wave's
+// lanes are shared out to its asking nodes instead, 64 / next_pow2(nodes)
+// lanes to each, which take the samples in turn (26 us).
+__device__ __forceinline__ int nearest_sample(const Tool &t, bool need, double px, double py, double pz) {
+    const unsigned long long m = __ballot(need);
+    if (!m) return -1;
+    const int lane = threadIdx.x % kWave;
+    const int na = __popcll(m);
+    int L = kWave;  // lanes per node
+    for (int c = 1; c < na; c *= 2) L /= 2;
+    int src = lane, q = 0;
+    for (unsigned long long b = m; b; b &= b - 1, ++q)
+        if (lane / L == q) src = __ffsll(b) - 1;
+    const double x = __shfl(px, src, kWave), y = __shfl(py, src, kWave), z = __shfl(pz, src, kWave);
+    double best = t.rc2;
+    int at = -1;
+    if (lane / L < na) {
+#pragma unroll 4
+        for (int s = lane % L; s < t.nsamples; s += L) {
+            const double dx = x - t.sx[s], dy = y - t.sy[s], dz = z - t.sz[s];
+            const double d2 = dx * dx + dy * dy + dz * dz;
+            if (d2 < best && d2 > 1e-20) { best = d2; at = s; }
+        }
+    }
+    for (int o = L / 2; o > 0; o /= 2) {
+        const double od = __shfl_xor(best, o, kWave);
+        const int oi = __shfl_xor(at, o, kWave);
+        if (oi >= 0 && (at < 0 || od < best || (od == best && oi < at))) { best = od; at = oi; }
+    }
+    const unsigned long long lt = lane ? (~0ull >> (64 - lane)) : 0ull;
+    const int hit = __shfl(at, __popcll(m & lt) * L % kWave, kWave);
+    return need ? hit : -1;
+}
+
 // mpmGridUpdateKernel, MPMWorkpieceSolver.cu:136-193 (point samples) and its
 // analytic-SDF form with tool velocity and Coulomb friction, for node
 // (i, j, k) = idx.  Takes the P2G sums c[] of the tile windows
 // (gather_tile_sums) and adds the accumulators when `tp` flags them,
 // zeroing what it has read; writes node velocity, mass and T*m.  When
 // `direct_T` is set (no diffusion pass follows) it also writes the gather
-// temperature.  Returns the node's contact-force contribution.
+// temperature.  `sample` is the point tool's nearest sample (nearest_sample).
+// Returns the node's contact-force contribution.
 template <typename R>
 __device__ __forceinline__ double grid_node(const GridView<R> &g, const Grid<R> &G, const TileParts<R> &tp,
                                             const Material<R> &M, const Tool &tool, R dt, int direct_T, int64_t idx,
-                                            int i, int j, int k, R c[8]) {
+                                            int i, int j, int k, int sample, R c[8]) {
     double cf = 0.0;
     {
         if (*tp.acc_flag) {
@@ -265,33 +305,19 @@ __device__ __forceinline__ double grid_node(const GridView<R> &g, const Grid<R> 
                 // node position nodePosition (:37-41), in FP64
                 const double px = g.ox + i * g.hd, py = g.oy + j * g.hd, pz = g.oz + k * g.hd;
                 if (tool.kind == kToolPoints) {
-                    if (px >= tool.lo[0] && px <= tool.hi[0] && py >= tool.lo[1] && py <= tool.hi[1] &&
-                        pz >= tool.lo[2] && pz <= tool.hi[2]) {
-                        double r2 = tool.rc2;
-                        double bdx = 0, bdy = 0, bdz = 0;
-                        bool hit = false;
-                        for (int s = 0; s < tool.nsamples; ++s) {
-                            double dx = px - tool.sx[s], dy = py - tool.sy[s], dz = pz - tool.sz[s];
-                            double d2 = dx * dx + dy * dy + dz * dz;
-                            if (d2 < r2 && d2 > 1e-20) {
-                                r2 = d2;
-                                bdx = dx; bdy = dy; bdz = dz;
-                                hit = true;
-                            }
-                        }
-                        if (hit) {
-                            double len = sqrt(bdx * bdx + bdy * bdy + bdz * bdz);
-                            R nx = R(0), ny = R(0), nz = R(0);
-                            if (len > 1e-12) { nx = (R)(bdx / len); ny = (R)(bdy / len); nz = (R)(bdz / len); }
-                            R vn = vx * nx + vy * ny + vz * nz;
-                            if (vn < R(0)) {
-                                cf += (double)fabs(mass * vn / rmax(dt, R(1e-15)));
-                                vx -= vn * nx; vy -= vn * ny; vz -= vn * nz;
-                                R heat = R(0.5) * mass * vn * vn * M.c_damp;
-                                R dT = heat / rmax(mass * M.cp, R(1e-12));
-                                if (M.clamp) dT = rmin(dT, M.dT_max);
-                                tm += dT * mass;
-                            }
+                    if (sample >= 0) {
+                        const double bdx = px - tool.sx[sample], bdy = py - tool.sy[sample], bdz = pz - tool.sz[sample];
+                        double len = sqrt(bdx * bdx + bdy * bdy + bdz * bdz);
+                        R nx = R(0), ny = R(0), nz = R(0);
+                        if (len > 1e-12) { nx = (R)(bdx / len); ny = (R)(bdy / len); nz = (R)(bdz / len); }
+                        R vn = vx * nx + vy * ny + vz * nz;
+                        if (vn < R(0)) {
+                            cf += (double)fabs(mass * vn / rmax(dt, R(1e-15)));
+                            vx -= vn * nx; vy -= vn * ny; vz -= vn * nz;
+                            R heat = R(0.5) * mass * vn * vn * M.c_damp;
+                            R dT = heat / rmax(mass * M.cp, R(1e-12));
+                            if (M.clamp) dT = rmin(dT, M.dT_max);
+                            tm += dT * mass;
                         }
                     }
                 } else if (tool.kind == kToolWedge || tool.kind == kToolVoxel ||
@@ -357,14 +383,26 @@ __device__ __forceinline__ void grid_update_block(const GridView<R> &g, const Gr
     // and the binning keys are 32-bit); the block size is any multiple of
     // the wave (the autotuner picks it)
     const int idx = blk * (int)blockDim.x + (int)threadIdx.x;
-    if (idx < g.nn) {
+    const bool node = idx < g.nn;
+    int i = 0, j = 0, k = 0;
+    R c[8];
+    if (node) {
         const int row = idx / g.nx;
-        const int i = idx - row * g.nx;
-        const int k = row / g.ny, j = row - k * g.ny;
-        R c[8];
+        i = idx - row * g.nx;
+        k = row / g.ny;
+        j = row - k * g.ny;
         gather_tile_sums(tp, i, j, k, c);
-        cf = grid_node(g, G, tp, M, tool, dt, direct_T, idx, i, j, k, c);
     }
+    int sample = -1;
+    if (tool.kind == kToolPoints) {  // uniform over the workgroup
+        // nodes in the samples' box (grown by r_c) that may be live
+        const double px = g.ox + i * g.hd, py = g.oy + j * g.hd, pz = g.oz + k * g.hd;
+        const bool need = node && k > g.kfix && (c[0] > R(1e-18) || *tp.acc_flag) && px >= tool.lo[0] &&
+                          px <= tool.hi[0] && py >= tool.lo[1] && py <= tool.hi[1] && pz >= tool.lo[2] &&
+                          pz <= tool.hi[2];
+        sample = nearest_sample(tool, need, px, py, pz);
+    }
+    if (node) cf = grid_node(g, G, tp, M, tool, dt, direct_T, idx, i, j, k, sample, c);
     // the contact force: one fixed-order partial per wave of 64 nodes, the
     // same partials for every block size and block order
     cf = wave_sum(cf);
