@@ -341,8 +341,10 @@ __device__ __forceinline__ void apic_g2p(const Particles<R> &P, int i, const G2P
 
 // One workgroup per tile: the APIC G2P and / or P2G of the tile's particles,
 // thread tid taking particles b0 + tid, b0 + tid + kBlock, ... (slot-major
-// order: consecutive particles sit in different cells).  The window goes to
-// tpart[t] (QN node records of 8 channels).  counters[0] counts particles whose
+// order: consecutive particles sit in different cells); of a tile shared by
+// `parts` workgroups each takes every parts-th run of kBlock particles and
+// stores a window of its own.  The window goes to tpart[block] (QN node
+// records of 8 channels).  counters[0] counts particles whose
 // stencil left the window, counters[2] is set when one was scattered into
 // the node accumulators.
 template <typename R, bool DO_G2P, bool DO_P2G, bool HAS_BACK>
@@ -350,7 +352,7 @@ __device__ __forceinline__ void apic_tile_block(const Particles<R> &P, const Gri
                                                 const Material<R> &M, R dt, double dtd, double zcut,
                                                 G2PFlags flags, double ref_temp, double *part,
                                                 const int32_t *cell_start, const TileGeom &tg, int32_t *counters,
-                                                R *tpart, int t) {
+                                                R *tpart, int block, int parts) {
     constexpr int kNodeBytes = DO_G2P ? QN * (int)sizeof(vec4_t<R>) : 0;
     constexpr int kAccBytes = DO_P2G ? 8 * QN * (int)sizeof(R) : 0;
     __shared__ __align__(32) unsigned char smem[kNodeBytes + kAccBytes + 32];
@@ -358,6 +360,7 @@ __device__ __forceinline__ void apic_tile_block(const Particles<R> &P, const Gri
     R *s_acc = DO_P2G ? reinterpret_cast<R *>(smem + kNodeBytes) : nullptr;
     const bool stats = DO_G2P && !DO_P2G && flags.stats != 0;
     const int tid = threadIdx.x, lane = tid % kWave;
+    const int t = block / parts, part0 = block - t * parts;
     const int tx = t % tg.ntx, ty = (t / tg.ntx) % tg.nty, tz = t / (tg.ntx * tg.nty);
     // window node 0 is the node before the tile's first cell
     const int qx0 = tg.ox + tx * TX - 1, qy0 = tg.oy + ty * TY - 1, qz0 = tg.oz + tz * TZ - 1;
@@ -385,7 +388,7 @@ __device__ __forceinline__ void apic_tile_block(const Particles<R> &P, const Gri
             for (int w = tid; w < 8 * QN; w += kBlock) s_acc[w] = R(0);
         __syncthreads();
         int my_oow = 0, my_acc = 0;
-        for (int i = b0 + tid; i < b1; i += kBlock) {
+        for (int i = b0 + part0 * kBlock + tid; i < b1; i += kBlock * parts) {
             PState<R> p;
             p.status = P.status[i];
             if (p.status == kInactive) continue;
@@ -433,8 +436,8 @@ __device__ __forceinline__ void apic_tile_block(const Particles<R> &P, const Gri
         }
         if (DO_P2G) {
             __syncthreads();  // every LDS atomic is in
-            if constexpr (sizeof(R) == 4) store_window_pairs(tpart + (int64_t)t * (8 * QN), s_acc, tid);
-            else store_window<R, QN>(tpart + (int64_t)t * (8 * QN), s_acc, tid);
+            if constexpr (sizeof(R) == 4) store_window_pairs(tpart + (int64_t)block * (8 * QN), s_acc, tid);
+            else store_window<R, QN>(tpart + (int64_t)block * (8 * QN), s_acc, tid);
         }
         int cntv = my_oow, cnta = my_acc;
 #pragma unroll
@@ -445,9 +448,9 @@ __device__ __forceinline__ void apic_tile_block(const Particles<R> &P, const Gri
         if (lane == 0 && cntv) atomicAdd(counters, cntv);
         if (lane == 0 && cnta) atomicOr(counters + 2, 1);
     } else if (DO_P2G) {
-        zero_window<R, QN>(tpart + (int64_t)t * (8 * QN), tid);
+        zero_window<R, QN>(tpart + (int64_t)block * (8 * QN), tid);
     }
-    if (stats) block_reduce_stats(st, part, t);
+    if (stats) block_reduce_stats(st, part, block);
 }
 
 template <typename R, bool DO_G2P, bool DO_P2G, bool HAS_BACK>
@@ -457,7 +460,8 @@ __global__ void __launch_bounds__(kBlock) k_apic_tile_batch(const TileWork<R> *_
     const int w = find_item(items, nitems, b);
     const TileWork<R> &W = items[w];
     apic_tile_block<R, DO_G2P, DO_P2G, HAS_BACK>(W.P, W.g, W.G, W.M, W.dt, W.dtd, W.zcut, W.flags, W.ref_temp,
-                                                 W.part, W.cell_start, W.tg, W.counters, W.tpart, b - W.block0);
+                                                 W.part, W.cell_start, W.tg, W.counters, W.tpart, b - W.block0,
+                                                 W.parts);
 }
 
 // The loose particles of the APIC pass, one thread each, nodes read from

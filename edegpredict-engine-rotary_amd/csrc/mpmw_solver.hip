@@ -760,6 +760,37 @@ void free_sort_state(mpmw_solver *s) {
     S = SortState();
 }
 
+// The tiles that hold particles (the grid has 4 cells around them).
+int64_t occupied_tiles(const mpmw_solver *s) {
+    auto tiles = [](int n, int T) -> int64_t { return std::max(1, (n - 9 + T - 1) / T); };
+    return tiles(s->nx, TX) * tiles(s->ny, TY) * tiles(s->nz, TZ);
+}
+
+// Workgroups that share each tile of a launch of `tiles` occupied tiles.  A workgroup
+// walks its tile's slots (8 in a slab) one after another, each a chain of
+// loads and dependent arithmetic, so a launch of fewer workgroups than the
+// chip holds at once (256 CUs, 2 each in FP32, 1 in FP64) takes as long as
+// one tile however small it is: 27 tiles (20 thousand particles) 56 us, 64
+// (131 thousand) 63 us.  Sharing a tile costs its prologue and its window
+// once more, so tiles are shared only while the launch then still fits the
+// chip in one go: 8 ways 18 us at 27 tiles, 8 ways 34 us at 64 (the grid
+// update, reading more windows, 9 -> 12 and 25 -> 27 us).  The
+// deterministic mode keeps one workgroup per tile: its sums must not depend
+// on what else is in the launch.  So does an FP32 workpiece under a point
+// tool: such a tool has no motion of its own, the workpiece moves through the
+// grid, and the nearly empty nodes along its moving surface turn the last
+// bits of their sums into velocity and contact heat (regrouping the sums
+// moved the temperatures of a 200-step pass by up to 5e-4, against 5e-7 under
+// a wedge or drill).
+constexpr int kMostParts = 8;
+int tile_sharing(const mpmw_solver *s, int64_t tiles) {
+    if (s->deterministic || (s->tool_kind == MPMW_TOOL_POINTS && !s->fp64)) return 1;
+    const int64_t resident = s->fp64 ? 256 : 512;
+    int p = 1;
+    while (p < kMostParts && tiles * p * 2 <= resident) p *= 2;
+    return p;
+}
+
 // Bin the particles into cell tiles of the current grid: stable radix sort
 // by tile-major cell key, slot-major order inside each tile, then one gather
 // of every particle field.  Only the order changes, never a value.
@@ -791,7 +822,8 @@ template <typename R> int sort_launch(mpmw_solver *s) {
         hipLaunchKernelGGL(k_fill<int32_t>, dim3(1), dim3(64), 0, s->stream, S.oow, (int64_t)3, 0);
     }
     {
-        const int64_t bytes = (int64_t)tg.ntiles * 8 * (s->apic ? QN : WN) * (int64_t)s->rsz;
+        S.most_parts = tile_sharing(s, occupied_tiles(s));
+        const int64_t bytes = (int64_t)tg.ntiles * S.most_parts * 8 * (s->apic ? QN : WN) * (int64_t)s->rsz;
         if (bytes > s->tpart_cap) {
             const int64_t c = std::max<int64_t>(bytes, s->tpart_cap * 5 / 4);
             dfree(s, s->tpart, (size_t)s->tpart_cap);
@@ -914,13 +946,13 @@ int loose_pass_t(mpmw_solver *s, double dt, double zcut, G2PFlags fl) {
     SortState &S = s->sort;
     if (s->apic) {
         hipLaunchKernelGGL((k_apic_loose<R, DO_G2P, DO_P2G, HAS_BACK>), dim3(nbl), dim3(kBlock), 0, s->stream, P, g,
-                           G, M, (R)dt, dt, zcut, fl, s->prm.ref_temp, s->part + (int64_t)S.geom.ntiles * kRed,
+                           G, M, (R)dt, dt, zcut, fl, s->prm.ref_temp, s->part + (int64_t)S.geom.ntiles * S.pass_parts * kRed,
                            S.loose_begin, S.loose_end, S.oow + 2);
         HIP_TRY(hipGetLastError());
         return MPMW_OK;
     }
     hipLaunchKernelGGL((k_loose<R, DO_G2P, DO_P2G && !DET, HAS_BACK>), dim3(nbl), dim3(kBlock), 0, s->stream, P, g,
-                       G, M, (R)dt, dt, zcut, fl, s->prm.ref_temp, s->part + (int64_t)S.geom.ntiles * kRed,
+                       G, M, (R)dt, dt, zcut, fl, s->prm.ref_temp, s->part + (int64_t)S.geom.ntiles * S.pass_parts * kRed,
                        S.loose_begin, S.loose_end, S.oow + 2);
     if (DET && DO_P2G)
         hipLaunchKernelGGL(k_loose_p2g_ordered<R>, dim3(1), dim3(kWave), 0, s->stream, P, g, G, S.loose_begin,
@@ -939,6 +971,7 @@ template <typename R, bool HAS_BACK> int det_p2g_pass(mpmw_solver *s, double dt,
     G2PFlags fl;
     fl.chip = 0;
     fl.stats = 0;
+    s->sort.win_parts = s->sort.pass_parts = 1;
     hipLaunchKernelGGL(k_fill<int32_t>, dim3(1), dim3(64), 0, s->stream, s->sort.oow + 1, (int64_t)2, 0);
     hipLaunchKernelGGL((k_tile<R, false, true, HAS_BACK, true>), dim3(tg.ntiles), dim3(kBlock), 0, s->stream,
                        pview<R>(s), gview<R>(s), grid_arrays<R>(s), material<R>(s), (R)dt, dt, zcut, fl,
@@ -995,6 +1028,7 @@ template <typename R> TileParts<R> tile_parts(const mpmw_solver *s) {
     tp.acc_flag = s->sort.oow + 2;
     tp.tg = s->sort.geom;
     tp.quad = s->apic ? 1 : 0;
+    tp.parts = s->sort.win_parts;
     return tp;
 }
 
@@ -1007,7 +1041,7 @@ template <typename R> int step_end(mpmw_solver *s, double dt, const StepPlan &sp
     s->snap_valid = s->snap_on;
     if (sp.fl.stats) {
         Timed t(s, MPMW_K_REDUCE);
-        if ((rc = finalize_stats(s, s->sort.geom.ntiles + loose_blocks(s)))) return rc;
+        if ((rc = finalize_stats(s, s->sort.geom.ntiles * s->sort.pass_parts + loose_blocks(s)))) return rc;
         s->stats_fresh = true;
         s->metrics_pending = true;
     } else {
@@ -2306,6 +2340,24 @@ template <typename R> void launch_tile_batch(hipStream_t stream, int variant, co
     }
 }
 
+// Grid-update variant of a member: point tool (1), tiles with more than one
+// window (2).
+constexpr int kGridVariants = 4;
+int grid_variant(const mpmw_solver *s) {
+    return (s->tool_kind == MPMW_TOOL_POINTS ? 1 : 0) + (s->sort.win_parts > 1 ? 2 : 0);
+}
+
+template <typename R> void launch_grid_batch(hipStream_t stream, int variant, const GridWork<R> *items, int n,
+                                             int blocks, int block, int order) {
+    const dim3 grid(blocks), blk(block);
+    switch (variant) {
+    case 0: hipLaunchKernelGGL((k_grid_update_batch<R, false, false>), grid, blk, 0, stream, items, n, order); break;
+    case 1: hipLaunchKernelGGL((k_grid_update_batch<R, true, false>), grid, blk, 0, stream, items, n, order); break;
+    case 2: hipLaunchKernelGGL((k_grid_update_batch<R, false, true>), grid, blk, 0, stream, items, n, order); break;
+    default: hipLaunchKernelGGL((k_grid_update_batch<R, true, true>), grid, blk, 0, stream, items, n, order); break;
+    }
+}
+
 // Tile-pass variant of a member: fused (0-3: backstress, deterministic) or
 // G2P-only before a rebuild (4-5: backstress); the APIC transfer's fused
 // (6-7) and G2P-only (8-9) passes; the standalone P2G of the step's begin
@@ -2505,9 +2557,9 @@ int graph_step(StepStaging &st, hipStream_t stream, size_t end, std::vector<uint
     return MPMW_OK;
 }
 
-// The tile-pass work item of a solver (blocks = its tiles; block0 is set by
-// the caller).
-template <typename R> TileWork<R> tile_work(mpmw_solver *s, double dt, double zcut, G2PFlags fl) {
+// The tile-pass work item of a solver in a launch of `tiles` occupied tiles in all
+// (block0 is set by the caller).
+template <typename R> TileWork<R> tile_work(mpmw_solver *s, double dt, double zcut, G2PFlags fl, int64_t tiles) {
     TileWork<R> t;
     t.P = pview<R>(s);
     t.g = gview<R>(s);
@@ -2524,7 +2576,8 @@ template <typename R> TileWork<R> tile_work(mpmw_solver *s, double dt, double zc
     t.counters = s->sort.oow;
     t.tpart = (R *)s->tpart;
     t.block0 = 0;
-    t.blocks = t.tg.ntiles;
+    t.parts = s->sort.pass_parts = std::min(tile_sharing(s, tiles), s->sort.most_parts);
+    t.blocks = t.tg.ntiles * t.parts;
     return t;
 }
 
@@ -2572,12 +2625,15 @@ template <typename R> int step_begin_many(mpmw_solver *const *members, size_t nm
     std::vector<TileWork<R>> pw[kTileVariants];
     std::vector<int> pm;
     int pblocks[kTileVariants] = {};
+    int64_t tiles = 0;
+    for (size_t m = 0; m < nm; ++m)
+        if (live[m] && !members[m]->p2g_ready) tiles += occupied_tiles(members[m]);
     for (size_t m = 0; m < nm; ++m) {
         if (!live[m]) continue;
         mpmw_solver *s = members[m];
         StepPlan &sp = plans[m];
         sp.zcut = s->tip[2] - s->h * 1.5;
-        if ((rc = ensure_part(s, s->sort.geom.ntiles + loose_blocks(s)))) return rc;
+        if ((rc = ensure_part(s, (int64_t)s->sort.geom.ntiles * s->sort.most_parts + loose_blocks(s)))) return rc;
         if (s->p2g_ready) continue;
         if (s->deterministic) {
             if ((rc = p2g_alone<R>(s, dts[m], sp.zcut))) return rc;
@@ -2588,7 +2644,8 @@ template <typename R> int step_begin_many(mpmw_solver *const *members, size_t nm
         if ((rc = zero_acc<R>(s))) return rc;
         hipLaunchKernelGGL(k_fill<int32_t>, dim3(1), dim3(64), 0, stream, s->sort.oow + 1, (int64_t)2, 0);
         const int v = p2g_variant(s);
-        TileWork<R> t = tile_work<R>(s, dts[m], sp.zcut, G2PFlags{});
+        TileWork<R> t = tile_work<R>(s, dts[m], sp.zcut, G2PFlags{}, tiles);
+        s->sort.win_parts = t.parts;
         t.block0 = pblocks[v];
         pblocks[v] += t.blocks;
         pw[v].push_back(t);
@@ -2626,7 +2683,7 @@ template <typename R> int step_begin_many(mpmw_solver *const *members, size_t nm
         mpmw_solver *s = members[m];
         StepPlan &sp = plans[m];
         // the binning may have changed in det_settle
-        if ((rc = ensure_part(s, s->sort.geom.ntiles + loose_blocks(s)))) return rc;
+        if ((rc = ensure_part(s, (int64_t)s->sort.geom.ntiles * s->sort.most_parts + loose_blocks(s)))) return rc;
         sp.diffusion = s->prm.specific_heat > 0.0 &&
                        s->prm.thermal_conductivity / (s->prm.density * s->prm.specific_heat) > 0.0;
         sp.alpha = sp.diffusion ? s->prm.thermal_conductivity / (s->prm.density * s->prm.specific_heat) : 0.0;
@@ -2687,9 +2744,14 @@ template <typename R> int step_many(mpmw_solver *const *members, size_t nm, cons
     std::vector<StepPlan> plans(nm);
     int rc;
     if ((rc = step_begin_many<R>(members, nm, dts, stream, st, plans))) return rc;
+    // the members that step, grouped by their grid-update variant
     std::vector<int> run;
-    for (size_t m = 0; m < nm; ++m)
-        if (plans[m].run) run.push_back((int)m);
+    int gitem[kGridVariants + 1] = {};   // a variant's first item
+    for (int v = 0; v < kGridVariants; ++v) {
+        for (size_t m = 0; m < nm; ++m)
+            if (plans[m].run && grid_variant(members[m]) == v) run.push_back((int)m);
+        gitem[v + 1] = (int)run.size();
+    }
     if (run.empty()) return MPMW_OK;
     const int nr = (int)run.size();
     // a tuning sample only on a step whose members all run the fused pass
@@ -2702,7 +2764,9 @@ template <typename R> int step_many(mpmw_solver *const *members, size_t nm, cons
     std::vector<GridWork<R>> gw(nr);
     std::vector<SumWork> sw(nr);
     std::vector<TileWork<R>> tw[kTileVariants];
-    int gblocks = 0, dblocks = 0, sblocks = 0, tblocks[kTileVariants] = {};
+    int gblocks[kGridVariants] = {}, dblocks = 0, sblocks = 0, tblocks[kTileVariants] = {};
+    int64_t tiles = 0;
+    for (int r = 0; r < nr; ++r) tiles += occupied_tiles(members[run[r]]);
     for (int r = 0; r < nr; ++r) {
         mpmw_solver *s = members[run[r]];
         const StepPlan &sp = plans[run[r]];
@@ -2718,11 +2782,12 @@ template <typename R> int step_many(mpmw_solver *const *members, size_t nm, cons
         g.direct_T = sp.diffusion ? 0 : 1;
         g.diffuse = sp.diffusion ? 1 : 0;
         g.force_part = s->fpart;
-        g.block0 = gblocks;
+        const int gv = grid_variant(s);
+        g.block0 = gblocks[gv];
         g.blocks = blocks_for(s->nn, cfg.grid_block);
         g.fwaves = (int32_t)((s->nn + kWave - 1) / kWave);
         g.pad_ = 0;
-        gblocks += g.blocks;
+        gblocks[gv] += g.blocks;
         g.dblock0 = dblocks;
         g.dblocks = blocks_for(s->nn, kDiffuseBlock);
         dblocks += g.dblocks;
@@ -2738,7 +2803,8 @@ template <typename R> int step_many(mpmw_solver *const *members, size_t nm, cons
         s->cf_chunks = sw[r].chunks;
         sw[r].counters = sp.next_rebuild ? nullptr : s->sort.oow;
         const int v = tile_variant(s, sp);
-        TileWork<R> t = tile_work<R>(s, dt, sp.zcut, sp.fl);
+        TileWork<R> t = tile_work<R>(s, dt, sp.zcut, sp.fl, tiles);
+        if (!sp.next_rebuild) s->sort.win_parts = t.parts;   // the grid item above reads the last P2G's windows
         t.block0 = tblocks[v];
         tblocks[v] += t.blocks;
         tw[v].push_back(t);
@@ -2769,8 +2835,10 @@ template <typename R> int step_many(mpmw_solver *const *members, size_t nm, cons
             if (ev) (void)hipEventRecord(ev[0], stream);
             {
                 Timed t(tm, MPMW_K_GRID);
-                hipLaunchKernelGGL(k_grid_update_batch<R>, dim3(gblocks), dim3(cfg.grid_block), 0, stream, d_gw, nr,
-                                   cfg.grid_order);
+                for (int v = 0; v < kGridVariants; ++v)
+                    if (gblocks[v] > 0)
+                        launch_grid_batch<R>(stream, v, d_gw + gitem[v], gitem[v + 1] - gitem[v], gblocks[v],
+                                             cfg.grid_block, cfg.grid_order);
             }
             if (ev) (void)hipEventRecord(ev[1], stream);
             {
@@ -2799,9 +2867,13 @@ template <typename R> int step_many(mpmw_solver *const *members, size_t nm, cons
         // kernel timing and tuning samples need events between the
         // launches: eager then
         if (st.graph_on && !(one && one->timing) && !sampling) {
-            std::vector<uint64_t> sig = {(uint64_t)nr, (uint64_t)gblocks, (uint64_t)dblocks, (uint64_t)off_sw,
+            std::vector<uint64_t> sig = {(uint64_t)nr, (uint64_t)dblocks, (uint64_t)off_sw,
                                          (uint64_t)cfg.tile_order, (uint64_t)cfg.grid_order,
                                          (uint64_t)cfg.grid_block, (uint64_t)cfg.post_order};
+            for (int v = 0; v < kGridVariants; ++v) {
+                sig.push_back((uint64_t)gitem[v + 1]);
+                sig.push_back((uint64_t)gblocks[v]);
+            }
             for (int v = 0; v < kTileVariants; ++v) {
                 sig.push_back((uint64_t)tw[v].size());
                 sig.push_back((uint64_t)tblocks[v]);

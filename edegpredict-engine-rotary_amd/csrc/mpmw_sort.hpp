@@ -76,4 +76,7 @@ struct SortState {
     int64_t steps_since = 0;           // steps since the out-of-window counter was reset
     int64_t sorts = 0;
     int64_t resorts = 0;               // re-binnings forced by the deterministic P2G
+    int32_t most_parts = 1;            // windows per tile that the window buffer has room for
+    int32_t win_parts = 1;             // windows per tile of the last P2G
+    int32_t pass_parts = 1;            // workgroups per tile of the last tile pass
 };

@@ -453,42 +453,51 @@ __device__ __forceinline__ void lds_add8(float *p, int stride, const float c[8],
     }
 }
 
-// Scatter of one particle whose stencil is not its home cell: through LDS
-// adds when the stencil lies in the tile window, else device atomics into
-// the node accumulators (then returns true).
+// Corner n of the scatter of one particle whose stencil is not its home
+// cell: through LDS adds when the stencil lies in the tile window, else
+// device atomics into the node accumulators (then returns true).
+template <typename R>
+__device__ __forceinline__ bool scatter_corner(const GridView<R> &g, gp<R> acc, R *s_acc, const Frac<R> &f, int wx0,
+                                               int wy0, int wz0, R mass, R vol, R vx, R vy, R vz, R T, const R s[6],
+                                               R fex, R fey, R fez, bool stress_force, bool ext_only, int n) {
+    const int lx = f.b[0] - wx0, ly = f.b[1] - wy0, lz = f.b[2] - wz0;
+    const bool in = s_acc && (unsigned)lx < (unsigned)TX && (unsigned)ly < (unsigned)TY && (unsigned)lz < (unsigned)TZ;
+    int64_t idx;
+    R w, gx, gy, gz;
+    if (!corner(g, f, n, idx, w, gx, gy, gz)) return !in;
+    R c[8];
+    const int nch = p2g_corner(mass, vol, vx, vy, vz, T, s, fex, fey, fez, stress_force, ext_only, w, gx, gy, gz, c);
+    if (in) {
+        lds_add8(s_acc + wnode(lx + (n & 1), ly + ((n >> 1) & 1), lz + ((n >> 2) & 1)), WN, c,
+                 nch == 8 ? 0xffu : 0x8fu);
+    } else {
+        R *a = acc + idx;
+        unsafeAtomicAdd(a, c[0]);
+        unsafeAtomicAdd(a + g.nn, c[1]);
+        unsafeAtomicAdd(a + 2 * g.nn, c[2]);
+        unsafeAtomicAdd(a + 3 * g.nn, c[3]);
+        unsafeAtomicAdd(a + 7 * g.nn, c[7]);
+        if (nch == 8) {
+            unsafeAtomicAdd(a + 4 * g.nn, c[4]);
+            unsafeAtomicAdd(a + 5 * g.nn, c[5]);
+            unsafeAtomicAdd(a + 6 * g.nn, c[6]);
+        }
+    }
+    return !in;
+}
+
+// All eight corners.
 template <typename R>
 __device__ __forceinline__ bool scatter_exception(const GridView<R> &g, gp<R> acc, R *s_acc, const Frac<R> &f,
                                                   int wx0, int wy0, int wz0, R mass, R vol, R vx, R vy, R vz, R T,
                                                   const R s[6], R fex, R fey, R fez, bool stress_force,
                                                   bool ext_only) {
-    const int lx = f.b[0] - wx0, ly = f.b[1] - wy0, lz = f.b[2] - wz0;
-    const bool in = s_acc && (unsigned)lx < (unsigned)TX && (unsigned)ly < (unsigned)TY && (unsigned)lz < (unsigned)TZ;
-    const int wb = wnode(lx, ly, lz);
-#pragma unroll
-    for (int n = 0; n < 8; ++n) {
-        int64_t idx;
-        R w, gx, gy, gz;
-        if (!corner(g, f, n, idx, w, gx, gy, gz)) continue;
-        R c[8];
-        const int nch = p2g_corner(mass, vol, vx, vy, vz, T, s, fex, fey, fez, stress_force, ext_only, w, gx, gy,
-                                   gz, c);
-        if (in) {
-            lds_add8(s_acc + wb + wnode(n & 1, (n >> 1) & 1, (n >> 2) & 1), WN, c, nch == 8 ? 0xffu : 0x8fu);
-        } else {
-            R *a = acc + idx;
-            unsafeAtomicAdd(a, c[0]);
-            unsafeAtomicAdd(a + g.nn, c[1]);
-            unsafeAtomicAdd(a + 2 * g.nn, c[2]);
-            unsafeAtomicAdd(a + 3 * g.nn, c[3]);
-            unsafeAtomicAdd(a + 7 * g.nn, c[7]);
-            if (nch == 8) {
-                unsafeAtomicAdd(a + 4 * g.nn, c[4]);
-                unsafeAtomicAdd(a + 5 * g.nn, c[5]);
-                unsafeAtomicAdd(a + 6 * g.nn, c[6]);
-            }
-        }
-    }
-    return !in;
+    bool out = false;
+#pragma unroll 1
+    for (int n = 0; n < 8; ++n)
+        out |= scatter_corner(g, acc, s_acc, f, wx0, wy0, wz0, mass, vol, vx, vy, vz, T, s, fex, fey, fez,
+                              stress_force, ext_only, n);
+    return out;
 }
 
 // The fields a P2G-only pass reads (mpmP2GKernel :103-133): velocity,
@@ -508,42 +517,91 @@ __device__ __forceinline__ void load_p2g_state(const Particles<R> &P, int i, PSt
     if (P.fx) { fex = P.fx[i]; fey = P.fy[i]; fez = P.fz[i]; }
 }
 
-template <typename R> __device__ __forceinline__ R shfl_from(R v, int src) { return __shfl(v, src, kWave); }
+// The value of the lane one before this one, zero in the first lane of each
+// 16 (DPP row_shr:1, a register move: no LDS round trip).
+__device__ __forceinline__ float lane_before(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x111, 0xf, 0xf, true));
+}
+__device__ __forceinline__ double lane_before(double v) {
+    const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)(unsigned)u, 0x111, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(unsigned)(u >> 32), 0x111, 0xf, 0xf, true);
+    return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned long long)(unsigned)lo);
+}
 
-// Combine the cell accumulators of a wave (an 8 x 8 layer of cells) into
-// node values of node layers z and z+1 and add them to the LDS window.
-// Node (x, y) of a layer = corner (0,0) of cell (x,y) + (1,0) of (x-1,y) +
-// (0,1) of (x,y-1) + (1,1) of (x-1,y-1); the far edge nodes x = 8 / y = 8
-// are formed by the lanes of the last column / row.  Fixed summation order.
-template <typename R>
-__device__ __forceinline__ void combine_layer(const CellAcc<R> &A, R *s_acc, int hx, int hy, int hz, int dz) {
-    const int lane = threadIdx.x % kWave;
+// Adds u[ch], then v[ch], to channel ch of the window node at a: the eight
+// reads, then the eight writes.  The lanes of the wave that call together
+// hold distinct nodes; the fence keeps the compiler from moving the next
+// call's reads, of nodes that other lanes write here, before these writes (a
+// wave's LDS operations complete in order).
+template <typename R> __device__ __forceinline__ void add_node(R *a, const R u[8], const R v[8]) {
+    R o[8];
+#pragma unroll
+    for (int ch = 0; ch < 8; ++ch) o[ch] = a[ch * WN];
+#pragma unroll
+    for (int ch = 0; ch < 8; ++ch) a[ch * WN] = (o[ch] + u[ch]) + v[ch];
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// Add the cell accumulators of a wave (an 8 x 8 layer of cells) to node
+// layer hz + DZ of the LDS window.  Node (x, y) takes corner (0, 0) of cell
+// (x, y), (1, 0) of (x - 1, y), (0, 1) of (x, y - 1) and (1, 1) of
+// (x - 1, y - 1), summed in that order; the layer's sum is added to what the
+// wave of the layer below has put there.  The cell before along x is the lane
+// before (a DPP move).  Layer hz is still empty, so along y a cell row simply
+// adds to node row y + 1 after node row y has its own; in layer hz + 1 the
+// row below comes by an LDS shuffle and its sum is added whole.  The last
+// column's and row's lanes add the far edges.  (A shuffle for each of the
+// five neighbour terms of a channel, each waited for, and single adds took
+// 4.2 us of a tile's 33 for the two layers; this takes 2.1.)
+template <typename R, int DZ>
+__device__ __forceinline__ void combine_layer(const CellAcc<R> &A, R *s_acc, int hx, int hy, int hz) {
+    R *a = s_acc + wnode(hx, hy, hz + DZ);
+    R b0[8], b1[8], zero[8], u[8], v[8];
 #pragma unroll
     for (int ch = 0; ch < 8; ++ch) {
-        const R c00 = A.v[ch][4 * dz + 0], c10 = A.v[ch][4 * dz + 1];
-        const R c01 = A.v[ch][4 * dz + 2], c11 = A.v[ch][4 * dz + 3];
-        const R l1 = shfl_from(c10, lane - 1);   // (x-1, y) corner (1,0)
-        const R l8 = shfl_from(c01, lane - 8);   // (x, y-1) corner (0,1)
-        const R l9 = shfl_from(c11, lane - 9);   // (x-1, y-1) corner (1,1)
-        const R e8 = shfl_from(c11, lane - 8);   // for node (8, y): (7, y-1) corner (1,1)
-        const R e1 = shfl_from(c11, lane - 1);   // for node (x, 8): (x-1, 7) corner (1,1)
-        R v = c00;
-        if (hx >= 1) v += l1;
-        if (hy >= 1) v += l8;
-        if (hx >= 1 && hy >= 1) v += l9;
-        R *a = s_acc + ch * WN;
-        a[wnode(hx, hy, hz + dz)] += v;
+        const R m0 = lane_before(A.v[ch][4 * DZ + 1]), m1 = lane_before(A.v[ch][4 * DZ + 3]);
+        b0[ch] = hx > 0 ? m0 : R(0);
+        b1[ch] = hx > 0 ? m1 : R(0);
+        zero[ch] = R(0);
+    }
+    if (DZ == 0) {
+#pragma unroll
+        for (int ch = 0; ch < 8; ++ch) { u[ch] = A.v[ch][0]; v[ch] = A.v[ch][2]; }
+        add_node(a, u, b0);
+        add_node(a + WX, v, b1);
         if (hx == TX - 1) {
-            R ve = c10;
-            if (hy >= 1) ve += e8;
-            a[wnode(TX, hy, hz + dz)] += ve;
+#pragma unroll
+            for (int ch = 0; ch < 8; ++ch) { u[ch] = A.v[ch][1]; v[ch] = A.v[ch][3]; }
+            add_node(a + 1, u, zero);
+            add_node(a + 1 + WX, v, zero);
         }
-        if (hy == TY - 1) {
-            R ve = c01;
-            if (hx >= 1) ve += e1;
-            a[wnode(hx, TY, hz + dz)] += ve;
+        return;
+    }
+    const int below = (int)(threadIdx.x % kWave) - TX;
+    R e[8];
+#pragma unroll
+    for (int ch = 0; ch < 8; ++ch) {
+        const R r01 = __shfl(A.v[ch][6], below, kWave), r11 = __shfl(b1[ch], below, kWave);
+        e[ch] = __shfl(A.v[ch][7], below, kWave);
+        u[ch] = A.v[ch][4] + b0[ch];
+        if (hy > 0) u[ch] = (u[ch] + r01) + r11;
+    }
+    add_node(a, u, zero);
+    if (hx == TX - 1) {
+#pragma unroll
+        for (int ch = 0; ch < 8; ++ch) u[ch] = A.v[ch][5] + (hy > 0 ? e[ch] : R(0));
+        add_node(a + 1, u, zero);
+    }
+    if (hy == TY - 1) {
+#pragma unroll
+        for (int ch = 0; ch < 8; ++ch) u[ch] = A.v[ch][6] + b1[ch];
+        add_node(a + WX, u, zero);
+        if (hx == TX - 1) {
+#pragma unroll
+            for (int ch = 0; ch < 8; ++ch) u[ch] = A.v[ch][7];
+            add_node(a + 1 + WX, u, zero);
         }
-        if (hx == TX - 1 && hy == TY - 1) a[wnode(TX, TY, hz + dz)] += c11;
     }
 }
 
@@ -557,8 +615,12 @@ __device__ __forceinline__ void combine_layer(const CellAcc<R> &A, R *s_acc, int
 // counters[1]; the caller re-bins and repeats the P2G when that count is not
 // zero.  Every sum then has a fixed order: per cell in slot order, across a
 // wave by the fixed shuffle tree, across tiles in tile order (k_grid_update_batch).
+// A tile may be shared by `parts` workgroups: workgroup p takes the slots p,
+// p + parts, ... and stores a window of its own (tile_sharing, mpmw_solver.hip,
+// says when).
 // Waves per SIMD the tile pass is compiled for (register budget 512 / waves).
-// FP32: 2 (a budget of 3 waves spills to scratch and measured 18 % slower);
+// FP32: 2 (with 3, and the stores made at once to fit 168 registers, 16.8 M
+// particles took 586 us against 544, 2 M particles 98 against 107);
 // FP64 keeps the compiler's choice.
 #ifndef MPMW_TILE_WAVES_F32
 #define MPMW_TILE_WAVES_F32 2
@@ -600,7 +662,7 @@ template <typename R, bool DO_G2P, bool DO_P2G, bool HAS_BACK, bool DET>
 __device__ __forceinline__ void tile_block(const Particles<R> &P, const GridView<R> &g, const Grid<R> &G,
                                            const Material<R> &M, R dt, double dtd, double zcut, G2PFlags flags,
                                            double ref_temp, double *part, const int32_t *cell_start,
-                                           const TileGeom &tg, int32_t *counters, R *tpart, int t) {
+                                           const TileGeom &tg, int32_t *counters, R *tpart, int block, int parts) {
     static_assert(TX == 8 && TY == 8 && TZ * TX * TY == kBlock, "one 8x8 cell layer per wave");
     constexpr int kNodeBytes = DO_G2P ? WN * (int)sizeof(vec4_t<R>) : 0;
     constexpr int kAccBytes = DO_P2G ? 8 * WN * (int)sizeof(R) : 0;
@@ -617,6 +679,7 @@ __device__ __forceinline__ void tile_block(const Particles<R> &P, const GridView
     // rebuild); the fused pass carries no statistics registers
     const bool stats = DO_G2P && !DO_P2G && flags.stats != 0;
     const int tid = threadIdx.x;
+    const int t = block / parts, part0 = block - t * parts;   // the tile, this workgroup's first slot
     const int lane = tid % kWave, wv = tid / kWave;
     const int hx = tid % TX, hy = (tid / TX) % TY, hz = tid / (TX * TY);
     const int tx = t % tg.ntx, ty = (t / tg.ntx) % tg.nty, tz = t / (tg.ntx * tg.nty);
@@ -632,7 +695,8 @@ __device__ __forceinline__ void tile_block(const Particles<R> &P, const GridView
     if (b0 < b1) {  // uniform over the workgroup
         // Prologue: the window's node records and the first slot's particle
         // inputs are requested before anything waits on them (the first
-        // slot is b0 + tid when the tile turns out uniform, else unused).
+        // slot is b0 + part0 * kBlock + tid when the tile turns out uniform,
+        // else unused).
         static_assert(WN <= 2 * kBlock, "two window records per thread");
         vec4_t<R> wrec[2];
         if (DO_G2P) {
@@ -645,7 +709,8 @@ __device__ __forceinline__ void tile_block(const Particles<R> &P, const GridView
             }
         }
         G2PIn<R> nxt;
-        if (DO_G2P) load_g2p_in(P, cnt > 0 && b0 + tid < b1 ? b0 + tid : b0, nxt);
+        const int i0 = b0 + part0 * kBlock + tid;
+        if (DO_G2P) load_g2p_in(P, cnt > part0 && i0 < b1 ? i0 : b0, nxt);
         if (DO_P2G) {
             for (int w = tid; w < 8 * WN; w += kBlock) s_acc[w] = R(0);
             if (tid == 0) s_qn = 0;  // before the count reduction's barrier
@@ -813,7 +878,7 @@ __device__ __forceinline__ void tile_block(const Particles<R> &P, const GridView
                 const bool ext_only = (p.status == kChip);
                 if (home_ok && f.b[0] == hgx && f.b[1] == hgy && f.b[2] == hgz) {
                     cell_accumulate(A, f, g.inv_h, mass, vol, p.vx, p.vy, p.vz, p.T, p.s, fex, fey, fez,
-                                    stress_force, ext_only, P.fx != nullptr);
+                                    stress_force, ext_only, !DO_G2P && P.fx != nullptr);
                 } else if (DET) {
                     ++my_exc;
                 } else {
@@ -839,9 +904,16 @@ __device__ __forceinline__ void tile_block(const Particles<R> &P, const GridView
                 }
             }
         };
-        int i_next = slot_index(0);
-        if (DO_G2P && !uniform) load_g2p_in(P, cnt > 0 ? i_next : b0, nxt);
-        for (int s = 0; s < maxc; ++s) {
+        // the index of slot `to`, slots from `from` on not yet passed (the
+        // prefix of an uneven tile runs over every slot)
+        auto slot_at = [&](int from, int to) -> int {
+            if (!uniform && !semi)
+                for (int s = from; s < to; ++s) (void)slot_index(s);
+            return slot_index(to);
+        };
+        int i_next = slot_at(0, part0);
+        if (DO_G2P && !uniform) load_g2p_in(P, cnt > part0 ? i_next : b0, nxt);
+        for (int s = part0; s < maxc; s += parts) {
             G2PIn<R> cur;
             if (DO_G2P) {
                 cur = nxt;
@@ -855,25 +927,27 @@ __device__ __forceinline__ void tile_block(const Particles<R> &P, const GridView
             }
             flush();
             const int i = i_next;
-            i_next = slot_index(s + 1);
-            if (DO_G2P) load_g2p_in(P, cnt > s + 1 ? i_next : b0, nxt);
+            i_next = slot_at(s + 1, s + parts);
+            if (DO_G2P) load_g2p_in(P, cnt > s + parts ? i_next : b0, nxt);
             process(cur, i, cnt > s);
         }
         flush();
         if (DO_P2G) {
             __syncthreads();  // exception atomics are in
-            combine_layer(A, s_acc, hx, hy, hz, 0);
+            combine_layer<R, 0>(A, s_acc, hx, hy, hz);
             __syncthreads();  // layer z written by wave z only
-            combine_layer(A, s_acc, hx, hy, hz, 1);
+            combine_layer<R, 1>(A, s_acc, hx, hy, hz);
             __syncthreads();  // layer z+1 written by wave z only
             if (!DET) {
-                // the queued particles, one per thread: their state as the
-                // G2P above stored it (the barriers order those stores
+                // the queued particles, a thread per corner (most tiles that
+                // queue any queue a few: the eight corners of a thread one
+                // after another took 8-11 us of such a tile, 33 in all; the
+                // corners side by side 2-3): their state as the G2P above stored it (the barriers order those stores
                 // before these loads); the external force was consumed by
                 // the G2P of a fused pass
                 const int nq = min(s_qn, kExcQueue);
                 if (nq > 0) {  // uniform over the workgroup
-                    for (int j = tid; j < nq; j += kBlock) {
+                    for (int j = tid / 8; j < nq; j += kBlock / 8) {
                         const int i = s_q[j];
                         PState<R> p;
                         p.status = P.status[i];
@@ -883,16 +957,16 @@ __device__ __forceinline__ void tile_block(const Particles<R> &P, const GridView
                         if (DO_G2P) fex = fey = fez = R(0);
                         const R mass = P.m ? P.m[i] : P.m0, vol = P.m ? P.V[i] : P.V0;
                         const Frac<R> f = base_and_frac(g, p.x, p.y, p.z);
-                        my_acc |= scatter_exception(g, G.acc, s_acc, f, wx0, wy0, wz0, mass, vol, p.vx, p.vy, p.vz,
-                                                    p.T, p.s, fex, fey, fez, p.status == kActive || p.status == kFixed,
-                                                    p.status == kChip)
+                        my_acc |= scatter_corner(g, G.acc, s_acc, f, wx0, wy0, wz0, mass, vol, p.vx, p.vy, p.vz, p.T,
+                                                 p.s, fex, fey, fez, p.status == kActive || p.status == kFixed,
+                                                 p.status == kChip, tid % 8)
                                       ? 1
                                       : 0;
                     }
                     __syncthreads();  // the queued scatters are in
                 }
             }
-            store_window<R, WN>(tpart + (int64_t)t * (8 * WN), s_acc, tid);
+            store_window<R, WN>(tpart + (int64_t)block * (8 * WN), s_acc, tid);
         }
         int cntv = my_oow, cnte = my_exc, cnta = my_acc;
 #pragma unroll
@@ -905,9 +979,9 @@ __device__ __forceinline__ void tile_block(const Particles<R> &P, const GridView
         if (DET && lane == 0 && cnte) atomicAdd(counters + 1, cnte);
         if (!DET && lane == 0 && cnta) atomicOr(counters + 2, 1);
     } else if (DO_P2G) {
-        zero_window<R, WN>(tpart + (int64_t)t * (8 * WN), tid);
+        zero_window<R, WN>(tpart + (int64_t)block * (8 * WN), tid);
     }
-    if (stats) block_reduce_stats(st, part, t);
+    if (stats) block_reduce_stats(st, part, block);
 }
 
 template <typename R, bool DO_G2P, bool DO_P2G, bool HAS_BACK, bool DET>
@@ -915,11 +989,11 @@ __global__ void __launch_bounds__(kBlock, TileWaves<R>::value)
     k_tile(Particles<R> P, GridView<R> g, Grid<R> G, Material<R> M, R dt, double dtd, double zcut, G2PFlags flags,
            double ref_temp, double *part, const int32_t *cell_start, TileGeom tg, int32_t *counters, R *tpart) {
     tile_block<R, DO_G2P, DO_P2G, HAS_BACK, DET>(P, g, G, M, dt, dtd, zcut, flags, ref_temp, part, cell_start, tg,
-                                                 counters, tpart, (int)blockIdx.x);
+                                                 counters, tpart, (int)blockIdx.x, 1);
 }
 
 // The tile pass of many solvers in one launch (see find_item): item w's
-// tiles are blocks [block0, block0 + ntiles).
+// tiles are blocks [block0, block0 + ntiles * parts), `parts` to a tile.
 template <typename R> struct TileWork {
     Particles<R> P;
     GridView<R> g;
@@ -933,7 +1007,7 @@ template <typename R> struct TileWork {
     TileGeom tg;
     int32_t *counters;
     R *tpart;
-    int32_t block0, blocks;
+    int32_t block0, blocks, parts;
 };
 
 template <typename R, bool DO_G2P, bool DO_P2G, bool HAS_BACK, bool DET>
@@ -947,7 +1021,7 @@ __global__ void __launch_bounds__(kBlock, TileWaves<R>::value)
     const int w = find_item(items, nitems, b);
     const TileWork<R> &W = items[w];
     tile_block<R, DO_G2P, DO_P2G, HAS_BACK, DET>(W.P, W.g, W.G, W.M, W.dt, W.dtd, W.zcut, W.flags, W.ref_temp, W.part,
-                                                 W.cell_start, W.tg, W.counters, W.tpart, b - W.block0);
+                                                 W.cell_start, W.tg, W.counters, W.tpart, b - W.block0, W.parts);
 }
 
 // ------------------------------------------------------ loose particles --
