@@ -29,6 +29,8 @@ template <typename R> struct Particles {
     R *v[3], *ef[3], *m, *V, *T;
     R *F[9], *Fp[9], *C[9], *s[6], *a[6];   // F and Fp hold H = F - I and Hp = Fp - I
     R *eps, *rate, *dmg, *sres;
+    // in the step: ef[0] null when every external force is zero, a[0] when
+    // every backstress is
     int32_t *id, *status, *lod;
     int32_t n;
 };
@@ -308,7 +310,7 @@ __device__ __forceinline__ void constitutive(const Particles<R> &P, int i, const
     s[0] -= tr / R(3); s[4] -= tr / R(3); s[8] -= tr / R(3);
     R al[6];
 #pragma unroll
-    for (int c = 0; c < 6; ++c) al[c] = P.a[c][i];
+    for (int c = 0; c < 6; ++c) al[c] = P.a[0] ? P.a[c][i] : R(0);
     const R ex = s[0] - al[0], ey = s[4] - al[1], ez = s[8] - al[2];
     const R exy = s[1] - al[3], exz = s[2] - al[4], eyz = s[5] - al[5];
     const R q = sqrt(R(1.5) * (ex * ex + ey * ey + ez * ez + R(2) * (exy * exy + exz * exz + eyz * eyz)));
@@ -398,7 +400,7 @@ __device__ __forceinline__ void constitutive(const Particles<R> &P, int i, const
                     P.sres[i] = fmax(P.sres[i], vm);
                 }
                 if (D >= M.dth) {
-                    P.status[i] = kChip;
+                    __hip_atomic_store(P.status + i, kChip, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                     skip = true;
                 }
             }
@@ -421,53 +423,52 @@ template <int D> __device__ __forceinline__ double row_shr(double v) {
     return __builtin_bit_cast(double, ((unsigned long long)(unsigned)hi << 32) | (unsigned long long)(unsigned)lo);
 }
 
-// One step of the segmented row sum over a particle's 7 channel values:
+// One step of the segmented row sum over a particle's NC channel values:
 // ch[q] += mk * (ch[q] of lane l - D in the same 16-lane row), zero from
 // before the row's start.  FP32: one v_fmac_f32 per channel reading its
 // first operand through DPP row_shr:D (the compiler's form is a DPP move,
-// the multiply-add and a wait state: three issue slots); the s_nop ahead of
-// the seven covers the wait states a DPP read needs after a VALU write of
-// its source and after an EXEC write, whatever the compiler placed before.
-// The same fused multiply-adds as the compiler's form, so the same sums.
-template <int D, typename R> __device__ __forceinline__ void seg_step(R (&ch)[7], R mk) {
+// the multiply-add and a wait state: three issue slots); the s_nop ahead
+// covers the wait states a DPP read needs after a VALU write of its source
+// and after an EXEC write, whatever the compiler placed before.  The same
+// fused multiply-adds as the compiler's form, so the same sums.
+template <int D, typename R, int NC> __device__ __forceinline__ void seg_step(R (&ch)[NC], R mk) {
+    if constexpr (sizeof(R) == 8) {
 #pragma unroll
-    for (int q = 0; q < 7; ++q) ch[q] = fma(row_shr<D>(ch[q]), mk, ch[q]);
-}
-#define MPMS_SEG_STEP_F32(D)                                                                                   \
-    template <> __device__ __forceinline__ void seg_step<D, float>(float (&ch)[7], float mk) {                  \
-        asm("s_nop 4\n\t"                                                                                       \
-            "v_fmac_f32_dpp %0, %0, %7 row_shr:" #D " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"               \
-            "v_fmac_f32_dpp %1, %1, %7 row_shr:" #D " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"               \
-            "v_fmac_f32_dpp %2, %2, %7 row_shr:" #D " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"               \
-            "v_fmac_f32_dpp %3, %3, %7 row_shr:" #D " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"               \
-            "v_fmac_f32_dpp %4, %4, %7 row_shr:" #D " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"               \
-            "v_fmac_f32_dpp %5, %5, %7 row_shr:" #D " row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"               \
-            "v_fmac_f32_dpp %6, %6, %7 row_shr:" #D " row_mask:0xf bank_mask:0xf bound_ctrl:1"                     \
-            : "+v"(ch[0]), "+v"(ch[1]), "+v"(ch[2]), "+v"(ch[3]), "+v"(ch[4]), "+v"(ch[5]), "+v"(ch[6])         \
-            : "v"(mk));                                                                                         \
+        for (int q = 0; q < NC; ++q) ch[q] = fma(row_shr<D>(ch[q]), mk, ch[q]);
+    } else if constexpr (NC == 4) {
+        asm("s_nop 4\n\t"
+            "v_fmac_f32_dpp %0, %0, %4 row_shr:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+            "v_fmac_f32_dpp %1, %1, %4 row_shr:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+            "v_fmac_f32_dpp %2, %2, %4 row_shr:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+            "v_fmac_f32_dpp %3, %3, %4 row_shr:%5 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+            : "+v"(ch[0]), "+v"(ch[1]), "+v"(ch[2]), "+v"(ch[3])
+            : "v"(mk), "n"(D));
+    } else {
+        static_assert(NC == 3, "three or four channels");
+        asm("s_nop 4\n\t"
+            "v_fmac_f32_dpp %0, %0, %3 row_shr:%4 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+            "v_fmac_f32_dpp %1, %1, %3 row_shr:%4 row_mask:0xf bank_mask:0xf bound_ctrl:1\n\t"
+            "v_fmac_f32_dpp %2, %2, %3 row_shr:%4 row_mask:0xf bank_mask:0xf bound_ctrl:1"
+            : "+v"(ch[0]), "+v"(ch[1]), "+v"(ch[2])
+            : "v"(mk), "n"(D));
     }
-MPMS_SEG_STEP_F32(1)
-MPMS_SEG_STEP_F32(2)
-MPMS_SEG_STEP_F32(4)
-MPMS_SEG_STEP_F32(8)
-#undef MPMS_SEG_STEP_F32
+}
 
-// Eight channel values as one record (two 16-byte or 32-byte accesses).
-__device__ __forceinline__ void store_record(float *p, const float v[8]) {
+// Four channel values as one record (16- or 32-byte accesses).
+__device__ __forceinline__ void store_record(float *p, const float v[4]) {
     reinterpret_cast<float4 *>(p)[0] = make_float4(v[0], v[1], v[2], v[3]);
-    reinterpret_cast<float4 *>(p)[1] = make_float4(v[4], v[5], v[6], v[7]);
 }
-__device__ __forceinline__ void store_record(double *p, const double v[8]) {
+__device__ __forceinline__ void store_record(double *p, const double v[4]) {
 #pragma unroll
-    for (int h = 0; h < 8; h += 2) reinterpret_cast<double2 *>(p)[h / 2] = make_double2(v[h], v[h + 1]);
+    for (int h = 0; h < 4; h += 2) reinterpret_cast<double2 *>(p)[h / 2] = make_double2(v[h], v[h + 1]);
 }
-__device__ __forceinline__ void load_record(const float *p, float v[8]) {
-    const float4 a = reinterpret_cast<const float4 *>(p)[0], b = reinterpret_cast<const float4 *>(p)[1];
-    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+__device__ __forceinline__ void load_record(const float *p, float v[4]) {
+    const float4 a = reinterpret_cast<const float4 *>(p)[0];
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
 }
-__device__ __forceinline__ void load_record(const double *p, double v[8]) {
+__device__ __forceinline__ void load_record(const double *p, double v[4]) {
 #pragma unroll
-    for (int h = 0; h < 8; h += 2) {
+    for (int h = 0; h < 4; h += 2) {
         const double2 a = reinterpret_cast<const double2 *>(p)[h / 2];
         v[h] = a.x; v[h + 1] = a.y;
     }
@@ -492,49 +493,67 @@ constexpr int kRounds = 3;   // window-add rounds of a wave's heads sharing a ba
 // three nodes at a time, heads sharing a base-node column in successive
 // rounds (a particle whose base node has left the tile since the sort adds
 // to the device grid directly).  The four windows'
-// sum is stored whole to tpart[t] (kWN records of 8 channels, the last
-// unused), which k_grid adds up: no device atomics for the window, whose
+// sum is stored whole to the workgroup's slot of tpart (kWN records of 4
+// channels), which k_grid adds up: no device atomics for the window, whose
 // nodes are mostly shared with neighbouring tiles (the device atomics were
 // 85 % of a per-particle form's time, and a window flush by atomics still a
 // third of this kernel's).
-template <typename R>
-__global__ void __launch_bounds__(kBlock) k_p2g(Particles<R> P, Grid<R> g, Mat<R> M, const StepArgs *__restrict__ sap,
-                                                const int32_t *__restrict__ tile_start, R *__restrict__ tpart) {
+//
+// The work of a tile is two jobs of their own, in workgroups of their own:
+// mass and momentum (JOB 0: needs v and C) and force (JOB 1: the LOD class,
+// the constitutive update and what it writes).  They share nothing but the
+// positions, read twice (24 of 230 bytes), and together they needed 234
+// registers and 68 KB of LDS a workgroup, two on a CU; each alone leaves
+// room for four: 16.5 M particles 1.40 -> 1.22 ms, and in FP64 (one on a CU
+// before, two now) 1.03 M particles 0.55 -> 0.37 ms.
+// A tile may be shared by `parts` workgroups of each job (chunks part, part +
+// parts, ...), each with a window of its own (p2g_parts, mpms_solver.hip).
+// FP32 / FP64: waves per SIMD the kernel is compiled for.
+template <typename R> struct P2GWaves { static constexpr int value = sizeof(R) == 4 ? 4 : 2; };
+
+template <typename R, int JOB>
+__device__ __forceinline__ void p2g_block(const Particles<R> &P, const Grid<R> &g, const Mat<R> &M,
+                                          const StepArgs *__restrict__ sap, const int32_t *__restrict__ tile_start,
+                                          R *__restrict__ dst, R *s_w, int32_t *s_own, int t, int part, int parts) {
     constexpr int kWaves = kBlock / 64;
-    __shared__ R s_w[kWaves * 7 * kWN];
-    __shared__ int32_t s_own[kWaves * kTX * kTY];   // per wave: the head owning a base-node column this round
+    constexpr int NC = JOB == 0 ? 4 : 3;   // channels: mass, momentum; force
     const StepArgs sa = *sap;
-    const int t = blockIdx.x;
     const int ts = tile_start[t], te = tile_start[t + 1];
     if (ts >= te) return;   // uniform over the workgroup
     const int ntx = (g.nb[0] + kTX - 1) / kTX, nty = (g.nb[1] + kTY - 1) / kTY;
     // the tile's first base node in lattice coordinates
     const int tx0 = g.lo[0] + (t % ntx) * kTX, ty0 = g.lo[1] + ((t / ntx) % nty) * kTY,
               tz0 = g.lo[2] + (t / (ntx * nty)) * kTZ;
-    for (int w = threadIdx.x; w < kWaves * 7 * kWN; w += kBlock) s_w[w] = R(0);
+    for (int w = threadIdx.x; w < kWaves * NC * kWN; w += kBlock) s_w[w] = R(0);
     __syncthreads();
     const int lane = threadIdx.x & 63;
-    R *const s_wave = s_w + (threadIdx.x / 64) * (7 * kWN);
+    R *const s_wave = s_w + (threadIdx.x / 64) * (NC * kWN);
     int missed = 0;
-    for (int c0 = ts; c0 < te; c0 += kBlock) {   // uniform over the workgroup
+    for (int c0 = ts + part * kBlock; c0 < te; c0 += kBlock * parts) {   // uniform over the workgroup
     const int i = c0 + threadIdx.x;
     bool live = i < te;
-    int32_t st = live ? P.status[i] : kInactive;
+    // the force job may be writing this particle's status: INACTIVE (which
+    // the test below finds for itself) or CHIP (no matter here)
+    int32_t st = kInactive;
+    if (live) st = JOB == 0 ? __hip_atomic_load(P.status + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : P.status[i];
     live = live && st != kInactive;
     double x = 0, y = 0, z = 0;
+    int32_t lod = kLodFar;
     if (live) {
         x = P.x[i]; y = P.y[i]; z = P.z[i];
-        int32_t lod = P.lod[i];
-        if (sa.lod_enabled && (st == kActive || st == kChip)) {
+        if (JOB == 1 && sa.lod_enabled && (st == kActive || st == kChip)) {
             const double dx = x - sa.tool[0], dy = y - sa.tool[1], dz = z - sa.tool[2];
             const double d = sqrt(dx * dx + dy * dy + dz * dz);
+            const int32_t was = P.lod[i];
             lod = d <= sa.lod_active ? kLodActive : (d <= sa.lod_near ? kLodNear : kLodFar);
-            P.lod[i] = lod;
+            if (lod != was) P.lod[i] = lod;
+        } else if (JOB == 1) {
+            lod = P.lod[i];
         }
         const int cx = (int)floor((x - g.ox) * g.inv_dx), cy = (int)floor((y - g.oy) * g.inv_dx),
                   cz = (int)floor((z - g.oz) * g.inv_dx);
         if (cx < 1 || cx >= g.dims[0] - 2 || cy < 1 || cy >= g.dims[1] - 2 || cz < 1 || cz >= g.dims[2] - 2) {
-            P.status[i] = kInactive;
+            if (JOB == 1) __hip_atomic_store(P.status + i, kInactive, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             live = false;
         }
     }
@@ -550,17 +569,22 @@ __global__ void __launch_bounds__(kBlock) k_p2g(Particles<R> P, Grid<R> g, Mat<R
     for (int c = 0; c < 9; ++c) C[c] = R(0);
     int key = -1 - lane;   // a run of its own unless live
     if (live) {
-        skip = P.lod[i] == kLodFar || fixed || st == kChip;
-        if (!skip && st == kActive) constitutive<R>(P, i, M, sig, J, skip, sa.islands);
+        if (JOB == 1) {
+            skip = lod == kLodFar || fixed || st == kChip;
+            if (!skip && st == kActive) constitutive<R>(P, i, M, sig, J, skip, sa.islands);
+        }
         ax = axis_weights<R>(x - g.ox, g.inv_dx);
         ay = axis_weights<R>(y - g.oy, g.inv_dx);
         az = axis_weights<R>(z - g.oz, g.inv_dx);
-        m = P.m[i];
-        VJ = P.V[i] * J;
-        vx = P.v[0][i]; vy = P.v[1][i]; vz = P.v[2][i];
-        efx = P.ef[0][i]; efy = P.ef[1][i]; efz = P.ef[2][i];
+        if (JOB == 0) {
+            m = P.m[i];
+            vx = P.v[0][i]; vy = P.v[1][i]; vz = P.v[2][i];
 #pragma unroll
-        for (int c = 0; c < 9; ++c) C[c] = P.C[c][i];
+            for (int c = 0; c < 9; ++c) C[c] = P.C[c][i];
+        } else {
+            VJ = P.V[i] * J;
+            if (P.ef[0]) { efx = P.ef[0][i]; efy = P.ef[1][i]; efz = P.ef[2][i]; }
+        }
         key = (az.b * g.dims[1] + ay.b) * g.dims[0] + ax.b;
     } else {
 #pragma unroll
@@ -620,8 +644,8 @@ __global__ void __launch_bounds__(kBlock) k_p2g(Particles<R> P, Grid<R> g, Mat<R
     static_assert(kRounds == 3, "round count");
     // particles whose run goes to the device grid (the host re-sorts when
     // they grow)
-    if (head && !lds_ok) atomicAdd(sa.islands + 2, (unsigned long long)(lane - seg_start + 1));
-    if (head) {
+    if (JOB == 0 && head && !lds_ok) atomicAdd(sa.islands + 2, (unsigned long long)(lane - seg_start + 1));
+    if (JOB == 0 && head) {
         // the run's stencil visits outside the sub-box: 27 less the product
         // of the stencil's in-box node counts per axis
         auto inbox = [&](int b0, int ax_) {
@@ -637,7 +661,7 @@ __global__ void __launch_bounds__(kBlock) k_p2g(Particles<R> P, Grid<R> g, Mat<R
     for (int a = 0; a < 3; ++a)
 #pragma unroll
         for (int b = 0; b < 3; ++b) {
-            R ch[3][7];
+            R ch[3][NC];
 #pragma unroll
             for (int c = 0; c < 3; ++c) {
                 const int gx = ax.b + a, gy = ay.b + b, gz = az.b + c;
@@ -647,22 +671,25 @@ __global__ void __launch_bounds__(kBlock) k_p2g(Particles<R> P, Grid<R> g, Mat<R
                 const R wgz = ax.w[a] * ay.w[b] * az.dw[c];
                 const R dpx = (R)((gx * g.dx + g.ox) - x), dpy = (R)((gy * g.dx + g.oy) - y),
                         dpz = (R)((gz * g.dx + g.oz) - z);
-                const R wm = w * mm;
                 R *const h = ch[c];
-                h[0] = w * m;
-                h[1] = wm * (pvx + C[0] * dpx + C[1] * dpy + C[2] * dpz);
-                h[2] = wm * (pvy + C[3] * dpx + C[4] * dpy + C[5] * dpz);
-                h[3] = wm * (pvz + C[6] * dpx + C[7] * dpy + C[8] * dpz);
-                h[4] = w * efx; h[5] = w * efy; h[6] = w * efz;
-                if (!skip) {
-                    h[4] += -VJ * (sig[0] * wgx + sig[1] * wgy + sig[2] * wgz);
-                    h[5] += -VJ * (sig[3] * wgx + sig[4] * wgy + sig[5] * wgz);
-                    h[6] += -VJ * (sig[6] * wgx + sig[7] * wgy + sig[8] * wgz);
+                if constexpr (JOB == 0) {
+                    const R wm = w * mm;
+                    h[0] = w * m;
+                    h[1] = wm * (pvx + C[0] * dpx + C[1] * dpy + C[2] * dpz);
+                    h[2] = wm * (pvy + C[3] * dpx + C[4] * dpy + C[5] * dpz);
+                    h[3] = wm * (pvz + C[6] * dpx + C[7] * dpy + C[8] * dpz);
+                } else {
+                    h[0] = w * efx; h[1] = w * efy; h[2] = w * efz;
+                    if (!skip) {
+                        h[0] += -VJ * (sig[0] * wgx + sig[1] * wgy + sig[2] * wgz);
+                        h[1] += -VJ * (sig[3] * wgx + sig[4] * wgy + sig[5] * wgz);
+                        h[2] += -VJ * (sig[6] * wgx + sig[7] * wgy + sig[8] * wgz);
+                    }
                 }
-                if (need[0]) seg_step<1, R>(ch[c], mk[0]);
-                if (need[1]) seg_step<2, R>(ch[c], mk[1]);
-                if (need[2]) seg_step<4, R>(ch[c], mk[2]);
-                if (need[3]) seg_step<8, R>(ch[c], mk[3]);
+                if (need[0]) seg_step<1>(ch[c], mk[0]);
+                if (need[1]) seg_step<2>(ch[c], mk[1]);
+                if (need[2]) seg_step<4>(ch[c], mk[2]);
+                if (need[3]) seg_step<8>(ch[c], mk[3]);
             }
             // the column's three nodes into the window (a node outside the
             // sub-box too: k_grid reads no window entry outside it)
@@ -671,15 +698,15 @@ __global__ void __launch_bounds__(kBlock) k_p2g(Particles<R> P, Grid<R> g, Mat<R
 #pragma unroll
                 for (int r = 0; r < kRounds; ++r) {
                     if (r < nrounds && myround == r) {
-                        R old[3][7];
+                        R old[3][NC];
 #pragma unroll
                         for (int c = 0; c < 3; ++c)
 #pragma unroll
-                            for (int k = 0; k < 7; ++k) old[c][k] = q[c * (kWX * kWY) + k * kWN];
+                            for (int k = 0; k < NC; ++k) old[c][k] = q[c * (kWX * kWY) + k * kWN];
 #pragma unroll
                         for (int c = 0; c < 3; ++c)
 #pragma unroll
-                            for (int k = 0; k < 7; ++k) q[c * (kWX * kWY) + k * kWN] = old[c][k] + ch[c][k];
+                            for (int k = 0; k < NC; ++k) q[c * (kWX * kWY) + k * kWN] = old[c][k] + ch[c][k];
                     }
                 }
             }
@@ -689,15 +716,18 @@ __global__ void __launch_bounds__(kBlock) k_p2g(Particles<R> P, Grid<R> g, Mat<R
                     const int64_t n = box_index(g, ax.b + a, ay.b + b, az.b + c);
                     if (n >= 0) {
                         const R *const h = ch[c];
-                        unsafeAtomicAdd(g.mass + n, h[0]);
-                        if (h[1] != R(0) || h[2] != R(0) || h[3] != R(0)) {
-                            unsafeAtomicAdd(g.p[0] + n, h[1]);
-                            unsafeAtomicAdd(g.p[1] + n, h[2]);
-                            unsafeAtomicAdd(g.p[2] + n, h[3]);
+                        if constexpr (JOB == 0) {
+                            unsafeAtomicAdd(g.mass + n, h[0]);
+                            if (h[1] != R(0) || h[2] != R(0) || h[3] != R(0)) {
+                                unsafeAtomicAdd(g.p[0] + n, h[1]);
+                                unsafeAtomicAdd(g.p[1] + n, h[2]);
+                                unsafeAtomicAdd(g.p[2] + n, h[3]);
+                            }
+                        } else {
+                            unsafeAtomicAdd(g.f[0] + n, h[0]);
+                            unsafeAtomicAdd(g.f[1] + n, h[1]);
+                            unsafeAtomicAdd(g.f[2] + n, h[2]);
                         }
-                        unsafeAtomicAdd(g.f[0] + n, h[4]);
-                        unsafeAtomicAdd(g.f[1] + n, h[5]);
-                        unsafeAtomicAdd(g.f[2] + n, h[6]);
                     }
                 }
             }
@@ -707,27 +737,44 @@ __global__ void __launch_bounds__(kBlock) k_p2g(Particles<R> P, Grid<R> g, Mat<R
     // the window, its waves' parts summed in wave order (entries of nodes
     // outside the sub-box are never read: their visits were counted as
     // missed)
-    R *const dst = tpart + (int64_t)t * (kWN * 8);
     for (int w = threadIdx.x; w < kWN; w += kBlock) {
-        R v[8];
+        R v[4] = {R(0), R(0), R(0), R(0)};
 #pragma unroll
-        for (int h = 0; h < 7; ++h) {
+        for (int h = 0; h < NC; ++h) {
             v[h] = s_w[h * kWN + w];
 #pragma unroll
-            for (int k = 1; k < kWaves; ++k) v[h] += s_w[(k * 7 + h) * kWN + w];
+            for (int k = 1; k < kWaves; ++k) v[h] += s_w[(k * NC + h) * kWN + w];
         }
-        v[7] = R(0);
-        store_record(dst + 8 * w, v);
+        store_record(dst + 4 * w, v);
     }
-    if (missed) atomicAdd(g.overflow, (unsigned long long)missed);
+    if (JOB == 0 && missed) atomicAdd(g.overflow, (unsigned long long)missed);
+}
+
+// Blocks 16 q + r and 16 q + r + 8 (r < 8) are the two jobs of window
+// 8 q + r: workgroups go to the 8 XCDs round-robin, so both jobs run on one
+// die and the second finds the tile's positions in its L2.  Window w is part
+// w % parts of tile w / parts; the mass and momentum records of the nw
+// windows come first in tpart, then the force records.
+template <typename R>
+__global__ void __launch_bounds__(kBlock, P2GWaves<R>::value)
+    k_p2g(Particles<R> P, Grid<R> g, Mat<R> M, const StepArgs *__restrict__ sap,
+          const int32_t *__restrict__ tile_start, R *__restrict__ tpart, int nw, int parts) {
+    __shared__ R s_w[(kBlock / 64) * 4 * kWN];
+    __shared__ int32_t s_own[(kBlock / 64) * kTX * kTY];   // per wave: the head owning a base-node column this round
+    const int w = (int)(blockIdx.x >> 4) * 8 + (int)(blockIdx.x & 7), job = (int)(blockIdx.x >> 3) & 1;
+    if (w >= nw) return;
+    const int t = w / parts;
+    R *const dst = tpart + ((int64_t)job * nw + w) * (kWN * 4);
+    if (job == 0) p2g_block<R, 0>(P, g, M, sap, tile_start, dst, s_w, s_own, t, w - t * parts, parts);
+    else p2g_block<R, 1>(P, g, M, sap, tile_start, dst, s_w, s_own, t, w - t * parts, parts);
 }
 
 // Adds the windows of the non-empty tiles whose window holds lattice node
 // (gx, gy, gz) (box coordinates i, j, k) to c[0..7): tile (tx, ty, tz) holds
 // nodes [kTX tx, kTX tx + kWX) x ... of the box, so at most two tiles per
-// axis, in a fixed order.
+// axis, in a fixed order; each tile's windows in order.
 template <typename R>
-__device__ __forceinline__ void gather_windows(const Grid<R> &g, const R *__restrict__ tpart,
+__device__ __forceinline__ void gather_windows(const Grid<R> &g, const R *__restrict__ tpart, int nw, int parts,
                                                const int32_t *__restrict__ tile_start, int i, int j, int k, R c[7]) {
     const int ntx = (g.nb[0] + kTX - 1) / kTX, nty = (g.nb[1] + kTY - 1) / kTY;
     const int x1 = i / kTX, y1 = j / kTY, z1 = k / kTZ;
@@ -740,10 +787,16 @@ __device__ __forceinline__ void gather_windows(const Grid<R> &g, const R *__rest
                 const int t = (tz * nty + ty) * ntx + tx;
                 if (tile_start[t] == tile_start[t + 1]) continue;   // an empty tile stores no window
                 const int w = ((k - kTZ * tz) * kWY + (j - kTY * ty)) * kWX + (i - kTX * tx);
-                R v[8];
-                load_record(tpart + ((int64_t)t * kWN + w) * 8, v);
+                const R *a = tpart + ((int64_t)t * parts * kWN + w) * 4;
+                for (int p = 0; p < parts; ++p, a += kWN * 4) {
+                    R v[4], f[4];
+                    load_record(a, v);
+                    load_record(a + (int64_t)nw * (kWN * 4), f);
 #pragma unroll
-                for (int h = 0; h < 7; ++h) c[h] += v[h];
+                    for (int h = 0; h < 4; ++h) c[h] += v[h];
+#pragma unroll
+                    for (int h = 0; h < 3; ++h) c[4 + h] += f[h];
+                }
             }
 }
 
@@ -781,7 +834,7 @@ template <typename R> __global__ void __launch_bounds__(kBlock) k_raster(Grid<R>
 // applyGridCollisionKernel (:475-492) on one node of the sub-box.
 template <typename R>
 __global__ void __launch_bounds__(kBlock) k_grid(Grid<R> g, const StepArgs *__restrict__ sap, const R *__restrict__ tpart,
-                                                 const int32_t *__restrict__ tile_start) {
+                                                 int nw, int parts, const int32_t *__restrict__ tile_start) {
     const StepArgs sa = *sap;
     const int64_t n = (int64_t)blockIdx.x * kBlock + threadIdx.x;
     if (n >= g.nn) return;
@@ -791,7 +844,7 @@ __global__ void __launch_bounds__(kBlock) k_grid(Grid<R> g, const StepArgs *__re
     R c[7] = {g.mass[n], g.p[0][n], g.p[1][n], g.p[2][n], g.f[0][n], g.f[1][n], g.f[2][n]};
     {
         const int i = (int)(n % g.nb[0]), j = (int)((n / g.nb[0]) % g.nb[1]), k = (int)(n / ((int64_t)g.nb[0] * g.nb[1]));
-        gather_windows(g, tpart, tile_start, i, j, k, c);
+        gather_windows(g, tpart, nw, parts, tile_start, i, j, k, c);
     }
     g.mass[n] = c[0];
     g.f[0][n] = c[4]; g.f[1][n] = c[5]; g.f[2][n] = c[6];
@@ -943,25 +996,28 @@ __device__ __forceinline__ void g2p_particle(const Particles<R> &P, const Grid<R
     } else if (st == kFixed) {
         P.v[0][i] = P.v[1][i] = P.v[2][i] = R(0);
     }
-    P.ef[0][i] = P.ef[1][i] = P.ef[2][i] = R(0);
+    if (P.ef[0]) P.ef[0][i] = P.ef[1][i] = P.ef[2][i] = R(0);
 }
 
 // One workgroup per base-node tile (the P2G's tiles): the tile's window of
 // node velocities and masses is read into LDS once, then its particles one
-// per thread in chunks.  Blocks from ntiles on take the particles after
-// every tile (INACTIVE at the sort: their external force is reset).
+// per thread in chunks; a tile may be shared by `parts` workgroups (chunks
+// part, part + parts, ...).  Blocks from ntiles * parts on take the particles
+// after every tile (INACTIVE at the sort: their external force is reset).
 template <typename R>
 __global__ void __launch_bounds__(kBlock) k_g2p(Particles<R> P, Grid<R> g, const StepArgs *__restrict__ sap, R dth,
-                                                const int32_t *__restrict__ tile_start, int ntiles, int tail_blocks) {
+                                                const int32_t *__restrict__ tile_start, int ntiles, int parts,
+                                                int tail_blocks) {
     const StepArgs sa = *sap;
-    const int t = blockIdx.x;
-    if (t >= ntiles) {   // uniform over the workgroup
-        for (int i = tile_start[ntiles] + (t - ntiles) * kBlock + (int)threadIdx.x; i < P.n; i += tail_blocks * kBlock)
+    const int tail = (int)blockIdx.x - ntiles * parts;
+    if (tail >= 0) {   // uniform over the workgroup
+        for (int i = tile_start[ntiles] + tail * kBlock + (int)threadIdx.x; i < P.n; i += tail_blocks * kBlock)
             g2p_particle<R>(P, g, sa, dth, i, nullptr, 0, 0, 0);
         return;
     }
     __shared__ NodeVM<R> s_n[kWN];
-    const int ts = tile_start[t], te = tile_start[t + 1];
+    const int t = (int)blockIdx.x / parts;
+    const int ts = tile_start[t] + ((int)blockIdx.x - t * parts) * kBlock, te = tile_start[t + 1];
     if (ts >= te) return;   // uniform over the workgroup
     const int ntx = (g.nb[0] + kTX - 1) / kTX, nty = (g.nb[1] + kTY - 1) / kTY;
     const int tx0 = g.lo[0] + (t % ntx) * kTX, ty0 = g.lo[1] + ((t / ntx) % nty) * kTY,
@@ -974,7 +1030,7 @@ __global__ void __launch_bounds__(kBlock) k_g2p(Particles<R> P, Grid<R> g, const
         s_n[w] = r;
     }
     __syncthreads();
-    for (int c0 = ts; c0 < te; c0 += kBlock) {
+    for (int c0 = ts; c0 < te; c0 += kBlock * parts) {
         const int i = c0 + (int)threadIdx.x;
         if (i < te) g2p_particle<R>(P, g, sa, dth, i, s_n, tx0, ty0, tz0);
     }

@@ -85,7 +85,9 @@ struct mpms_solver {
     // the P2G's base-node tiles: first particle of each (ntiles + 1)
     int32_t *tile_start = nullptr;
     int32_t ntiles = 0, tile_cap = 0;
-    void *tpart = nullptr;            // the tiles' P2G windows (kWN records of 8 channels each)
+    void *tpart = nullptr;            // the tiles' P2G windows (kWN records of 4 + 4 channels each)
+    int32_t p2g_parts = 1;            // P2G windows (workgroups of each job) per tile
+    bool has_ef = false, has_back = false;   // some external force / backstress may be nonzero
     int64_t tpart_cap = 0;            // bytes
     mpmw::ScratchBuf temp;
     // the step's scalars on the device (k_step_args) and its captured
@@ -245,6 +247,9 @@ int set_particles_impl(mpms_solver *s, const mpms_particle_arrays *a) {
         s->cap = n;
     }
     s->n = n;
+    s->has_ef = a->fext && std::any_of(a->fext, a->fext + 3 * (size_t)n, [](double v) { return v != 0.0; });
+    s->has_back = s->prm.kinematic_hardening > 0.0 ||
+                  (a->backstress && std::any_of(a->backstress, a->backstress + 6 * (size_t)n, [](double v) { return v != 0.0; }));
     int rc = 0;
     const std::vector<double> zero(std::max<int32_t>(n, 1) * 9, 0.0);
     std::vector<double> eye(std::max<int32_t>(n, 1) * 9, 0.0);
@@ -331,6 +336,20 @@ template <typename R> int stats(mpms_solver *s, double out[kStats]) {
     return MPMW_OK;
 }
 
+// Workgroups that share a tile in a pass of which `resident` workgroups run
+// at once.  A full tile holds 2048 particles, eight chunks of a workgroup one
+// after another, so a block of particles with fewer tiles than that takes as
+// long as one tile: 131 thousand particles (64 full tiles) shared 4 ways in
+// the P2G, 146 -> 58 us, and 8 ways in the G2P, 74 -> 26 us.
+// The tiles are counted as full ones, n / 2048: a box's edge tiles and its
+// margin hold few particles or none.
+int tile_sharing(const mpms_solver *s, int64_t resident) {
+    const int64_t tiles = s->n / (8 * kTX * kTY * kTZ) + 1;
+    int p = 1;
+    while (p < 8 && tiles * p * 2 <= resident) p *= 2;
+    return p;
+}
+
 // The grid fit (every kFitEvery steps): the overflow count of the last
 // interval must be zero; the sub-box covers every non-INACTIVE particle's
 // stencil plus kMargin nodes; the particles are sorted by base-node tile and
@@ -412,7 +431,9 @@ template <typename R> int fit(mpms_solver *s) {
             s->tile_cap = (int32_t)c;
         }
         s->ntiles = (int32_t)nt;
-        const int64_t tb = nt * (int64_t)kWN * 8 * (int64_t)s->rsz;
+        // the P2G's workgroups, two jobs a tile: four on a CU in FP32, two in FP64
+        s->p2g_parts = tile_sharing(s, s->fp64 ? 256 : 512);
+        const int64_t tb = nt * s->p2g_parts * (int64_t)kWN * 8 * (int64_t)s->rsz;
         if (tb > s->tpart_cap) {
             if (s->tpart) (void)hipFree(s->tpart);
             s->tpart = nullptr;
@@ -465,7 +486,9 @@ std::vector<uint64_t> graph_key(const mpms_solver *s) {
     std::vector<uint64_t> k = {(uint64_t)s->n, (uint64_t)s->nn, (uint64_t)s->nn_cap, (uint64_t)s->ntool,
                                (uint64_t)(uintptr_t)s->gblock, (uint64_t)(uintptr_t)s->d_tool_xyz,
                                (uint64_t)(uintptr_t)s->d_tool_vel, (uint64_t)(uintptr_t)s->d_sa,
-                               (uint64_t)s->ntiles, (uint64_t)(uintptr_t)s->tile_start,
+                               (uint64_t)s->ntiles, (uint64_t)s->p2g_parts,
+                               (uint64_t)(s->has_ef ? 1 : 0) | (uint64_t)(s->has_back ? 2 : 0),
+                               (uint64_t)(uintptr_t)s->tile_start,
                                (uint64_t)(uintptr_t)s->tpart};
     for (int a = 0; a < 3; ++a) k.push_back(((uint64_t)(uint32_t)s->lo[a] << 32) | (uint32_t)s->nb[a]);
     for (int f = 0; f < NFIELD; ++f) k.push_back((uint64_t)(uintptr_t)s->f[f]);
@@ -533,7 +556,11 @@ template <typename R> int step_impl(mpms_solver *s, double dt) {
         if ((double)out > kResortFraction * (double)s->n)
             if ((rc = fit<R>(s))) return rc;
     }
-    const Particles<R> P = pview<R>(s);
+    Particles<R> P = pview<R>(s);
+    // arrays of zeros are neither read nor cleared (24 and 24 bytes of the
+    // 500 a particle takes a step)
+    if (!s->has_ef) P.ef[0] = nullptr;
+    if (!s->has_back) P.a[0] = nullptr;
     const Grid<R> g = gview<R>(s);
     StepArgs sa;
     sa.dt = dt;
@@ -560,15 +587,17 @@ template <typename R> int step_impl(mpms_solver *s, double dt) {
                            s->stream, (uint32_t *)g.claim, s->nn);
         hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(kBlock), 0, s->stream, (uint32_t *)(s->d_counts + 1),
                            (int64_t)6);
-        hipLaunchKernelGGL(k_p2g<R>, dim3((unsigned)s->ntiles), dim3(kBlock), 0, s->stream, P, g, material<R>(s), dsa,
-                           (const int32_t *)s->tile_start, (R *)s->tpart);
+        const int pp = s->p2g_parts, nw = s->ntiles * pp;
+        hipLaunchKernelGGL(k_p2g<R>, dim3((unsigned)((nw + 7) / 8 * 16)), dim3(kBlock), 0, s->stream, P, g,
+                           material<R>(s), dsa, (const int32_t *)s->tile_start, (R *)s->tpart, nw, pp);
         if (s->ntool > 0)
             hipLaunchKernelGGL(k_raster<R>, dim3(blocks(s->ntool)), dim3(kBlock), 0, s->stream, g,
                                (const double *)s->d_tool_xyz, s->ntool);
         hipLaunchKernelGGL(k_grid<R>, dim3(blocks(s->nn)), dim3(kBlock), 0, s->stream, g, dsa, (const R *)s->tpart,
-                           (const int32_t *)s->tile_start);
-        hipLaunchKernelGGL(k_g2p<R>, dim3((unsigned)(s->ntiles + kTailBlocks)), dim3(kBlock), 0, s->stream, P, g, dsa,
-                           (R)s->prm.damage_threshold, (const int32_t *)s->tile_start, s->ntiles, kTailBlocks);
+                           nw, pp, (const int32_t *)s->tile_start);
+        const int gp = tile_sharing(s, 1024);
+        hipLaunchKernelGGL(k_g2p<R>, dim3((unsigned)(s->ntiles * gp + kTailBlocks)), dim3(kBlock), 0, s->stream, P, g,
+                           dsa, (R)s->prm.damage_threshold, (const int32_t *)s->tile_start, s->ntiles, gp, kTailBlocks);
     };
     if (!s->graph_on) {
         issue();
@@ -576,6 +605,7 @@ template <typename R> int step_impl(mpms_solver *s, double dt) {
     } else if ((rc = graph_step(s, issue))) {
         return rc;
     }
+    s->has_ef = false;   // the G2P has consumed it
     s->time += dt;
     s->step++;
     return MPMW_OK;
@@ -773,6 +803,7 @@ int mpms_apply_external_force(mpms_solver *s, const double c[3], double radius, 
     MS_CHECK(s);
     if (!c || !f) return fail(MPMW_E_INVAL, "null");
     if (s->n == 0 || std::sqrt(f[0] * f[0] + f[1] * f[1] + f[2] * f[2]) < 1e-12) return MPMW_OK;   // :1441
+    s->has_ef = true;
     if (s->fp64)
         hipLaunchKernelGGL(k_ext_force<double>, dim3(blocks(s->n)), dim3(kBlock), 0, s->stream, pview<double>(s), c[0],
                            c[1], c[2], radius, f[0], f[1], f[2]);
