@@ -20,6 +20,7 @@
 #include "mpmw_sort.hpp"
 #include "mpms_kernels.hpp"
 #include "mpms_internal.hpp"
+#include "mpmw_readback.hpp"
 
 namespace mpmw_internal {
 int set_error(int code, const std::string &msg);
@@ -217,22 +218,19 @@ int upload(mpms_solver *s, int k, const void *src, int32_t count, int comp = 1, 
     return MPMW_OK;
 }
 
-int download(mpms_solver *s, int k, void *dst, int32_t count, int comp = 1, int c = 0, double shift = 0.0) {
-    if (count <= 0 || !dst) return MPMW_OK;
-    if (k >= kFirstInt) {
-        MS_TRY(hipMemcpy(dst, s->f[k], sizeof(int32_t) * count, hipMemcpyDeviceToHost));
-        return MPMW_OK;
-    }
-    std::vector<double> t(count);
-    if (k <= Z || s->fp64) {
-        MS_TRY(hipMemcpy(t.data(), s->f[k], sizeof(double) * count, hipMemcpyDeviceToHost));
-    } else {
-        std::vector<float> u(count);
-        MS_TRY(hipMemcpy(u.data(), s->f[k], sizeof(float) * count, hipMemcpyDeviceToHost));
-        for (int32_t i = 0; i < count; ++i) t[i] = u[i];
-    }
-    for (int32_t i = 0; i < count; ++i) ((double *)dst)[(size_t)i * comp + c] = t[i] + shift;
-    return MPMW_OK;
+// Array dst of `comp` values a particle from fields k .. k + comp - 1 (null:
+// none); `eye` adds the identity (F and Fp are held less it).
+void read_field(const mpms_solver *s, std::vector<mpmw_internal::ReadArray> &out, int k, void *dst, int comp = 1,
+                bool eye = false) {
+    if (!dst) return;
+    mpmw_internal::ReadArray r;
+    r.dst = dst;
+    r.comp = comp;
+    r.kind = k >= kFirstInt ? mpmw_internal::kReadI32
+                            : (k <= Z || s->fp64 ? mpmw_internal::kReadF64 : mpmw_internal::kReadF32);
+    r.ones = eye ? 0x111u : 0u;
+    for (int c = 0; c < comp; ++c) r.src[c] = s->f[k + c];
+    out.push_back(r);
 }
 
 int set_particles_impl(mpms_solver *s, const mpms_particle_arrays *a) {
@@ -287,32 +285,26 @@ int set_particles_impl(mpms_solver *s, const mpms_particle_arrays *a) {
 int get_particles_impl(mpms_solver *s, mpms_particle_arrays *a) {
     MS_TRY(hipStreamSynchronize(s->stream));
     const int32_t n = std::min(a->n, s->n);
-    int rc = 0;
-    for (int c = 0; c < 3 && !rc; ++c) {
-        rc = download(s, X + c, a->pos, n, 3, c);
-        if (!rc) rc = download(s, VX + c, a->vel, n, 3, c);
-        if (!rc) rc = download(s, EFX + c, a->fext, n, 3, c);
-    }
-    if (!rc) rc = download(s, M, a->mass, n);
-    if (!rc) rc = download(s, V, a->volume, n);
-    if (!rc) rc = download(s, T, a->temperature, n);
-    for (int c = 0; c < 9 && !rc; ++c) {
-        const double id = (c % 4 == 0) ? 1.0 : 0.0;
-        rc = download(s, F0 + c, a->F, n, 9, c, id);
-        if (!rc) rc = download(s, FP0 + c, a->Fp, n, 9, c, id);
-        if (!rc) rc = download(s, C0 + c, a->C, n, 9, c);
-    }
-    for (int c = 0; c < 6 && !rc; ++c) {
-        rc = download(s, S0 + c, a->stress, n, 6, c);
-        if (!rc) rc = download(s, A0 + c, a->backstress, n, 6, c);
-    }
-    if (!rc) rc = download(s, EPS, a->plastic_strain, n);
-    if (!rc) rc = download(s, RATE, a->strain_rate, n);
-    if (!rc) rc = download(s, DMG, a->damage, n);
-    if (!rc) rc = download(s, SRES, a->residual_stress, n);
-    if (!rc) rc = download(s, ID, a->id, n);
-    if (!rc) rc = download(s, STATUS, a->status, n);
-    if (!rc) rc = download(s, LOD, a->lod, n);
+    std::vector<mpmw_internal::ReadArray> out;
+    read_field(s, out, X, a->pos, 3);
+    read_field(s, out, VX, a->vel, 3);
+    read_field(s, out, EFX, a->fext, 3);
+    read_field(s, out, M, a->mass);
+    read_field(s, out, V, a->volume);
+    read_field(s, out, T, a->temperature);
+    read_field(s, out, F0, a->F, 9, true);
+    read_field(s, out, FP0, a->Fp, 9, true);
+    read_field(s, out, C0, a->C, 9);
+    read_field(s, out, S0, a->stress, 6);
+    read_field(s, out, A0, a->backstress, 6);
+    read_field(s, out, EPS, a->plastic_strain);
+    read_field(s, out, RATE, a->strain_rate);
+    read_field(s, out, DMG, a->damage);
+    read_field(s, out, SRES, a->residual_stress);
+    read_field(s, out, ID, a->id);
+    read_field(s, out, STATUS, a->status);
+    read_field(s, out, LOD, a->lod);
+    const int rc = mpmw_internal::read_back(s->prm.device, s->stream, out, n);
     a->n = n;
     return rc;
 }
@@ -875,26 +867,18 @@ int mpms_get_grid(mpms_solver *s, int32_t lo[3], int32_t n[3], double *mass, dou
     for (int a = 0; a < 3; ++a) { lo[a] = s->lo[a]; n[a] = s->nb[a]; }
     if (!s->gblock || s->nn == 0) return MPMW_OK;
     MS_TRY(hipStreamSynchronize(s->stream));
-    const int64_t nn = s->nn, c = s->nn_cap;
-    std::vector<double> t((size_t)nn);
-    auto fetch = [&](int ch, double *dst, int comp, int k) -> int {
-        if (s->fp64) {
-            MS_TRY(hipMemcpy(t.data(), (double *)s->gblock + ch * c, sizeof(double) * nn, hipMemcpyDeviceToHost));
-        } else {
-            std::vector<float> u((size_t)nn);
-            MS_TRY(hipMemcpy(u.data(), (float *)s->gblock + ch * c, sizeof(float) * nn, hipMemcpyDeviceToHost));
-            for (int64_t i = 0; i < nn; ++i) t[i] = u[i];
-        }
-        for (int64_t i = 0; i < nn; ++i) dst[i * comp + k] = t[i];
-        return MPMW_OK;
-    };
-    int rc = 0;
-    if (mass) rc = fetch(0, mass, 1, 0);
-    for (int a = 0; a < 3 && !rc; ++a) {
-        if (mom) rc = fetch(1 + a, mom, 3, a);
-        if (!rc && force) rc = fetch(4 + a, force, 3, a);
+    // channels mass, momentum xyz, force xyz of the node block
+    const int64_t c = s->nn_cap * (int64_t)s->rsz;
+    std::vector<mpmw_internal::ReadArray> out(3);
+    double *const dst[3] = {mass, mom, force};
+    const int first[3] = {0, 1, 4}, comp[3] = {1, 3, 3};
+    for (int k = 0; k < 3; ++k) {
+        out[k].dst = dst[k];
+        out[k].comp = comp[k];
+        out[k].kind = s->fp64 ? mpmw_internal::kReadF64 : mpmw_internal::kReadF32;
+        for (int q = 0; q < comp[k]; ++q) out[k].src[q] = (const char *)s->gblock + (first[k] + q) * c;
     }
-    return rc;
+    return mpmw_internal::read_back(s->prm.device, s->stream, out, s->nn);
 }
 
 int mpms_get_diagnostics(mpms_solver *s, mpms_diagnostics *d) {

@@ -25,11 +25,13 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "mpmw.h"
 #include "mpmw_sdf.hpp"
 #include "mpmw_apic.hpp"
+#include "mpmw_readback.hpp"
 
 using namespace mpmw;
 
@@ -1171,6 +1173,76 @@ template <typename R> int download_field(mpmw_solver *s, int fld, double *dst, i
     return MPMW_OK;
 }
 
+// A part of one array on its way out: `count` rows from row i0 on, at byte
+// `at` of the chunk.
+struct ReadPiece {
+    const void *src[9];
+    int64_t i0;
+    uint64_t at;
+    int32_t count, comp, kind;
+    uint32_t ones;
+};
+constexpr int kReadPieces = 24;
+struct ReadTable {
+    ReadPiece p[kReadPieces];
+};
+
+__global__ void __launch_bounds__(kBlock) k_read_back(ReadTable t, char *out) {
+    const ReadPiece &p = t.p[blockIdx.y];
+    const int64_t ne = (int64_t)p.count * p.comp;
+    const int64_t stride = (int64_t)gridDim.x * kBlock;
+    for (int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x; e < ne; e += stride) {
+        if (p.kind == mpmw_internal::kReadI32) {
+            reinterpret_cast<int32_t *>(out + p.at)[e] = static_cast<const int32_t *>(p.src[0])[p.i0 + e];
+            continue;
+        }
+        const int64_t i = e / p.comp;
+        const int c = (int)(e - i * p.comp);
+        double v = p.kind == mpmw_internal::kReadF64 ? static_cast<const double *>(p.src[c])[p.i0 + i]
+                                                     : (double)static_cast<const float *>(p.src[c])[p.i0 + i];
+        if (p.ones >> c & 1u) v += 1.0;
+        reinterpret_cast<double *>(out + p.at)[e] = v;
+    }
+}
+
+// Host moves in parallel: (dst, src, bytes), src null for zeros.
+struct HostMove {
+    char *dst;
+    const char *src;
+    size_t bytes;
+};
+
+// The moves shared out in pieces of a megabyte among up to eight threads, one
+// for each two megabytes (most of the time of a move into fresh pageable
+// memory is its page faults, which threads take side by side).
+void move_out(const std::vector<HostMove> &moves) {
+    constexpr size_t kPiece = 1u << 20;
+    std::vector<HostMove> pieces;
+    size_t total = 0;
+    for (const HostMove &m : moves) {
+        total += m.bytes;
+        for (size_t o = 0; o < m.bytes; o += kPiece)
+            pieces.push_back({m.dst + o, m.src ? m.src + o : nullptr, std::min(kPiece, m.bytes - o)});
+    }
+    auto run = [&pieces](size_t first, size_t step) {
+        for (size_t k = first; k < pieces.size(); k += step) {
+            if (pieces[k].src) std::memcpy(pieces[k].dst, pieces[k].src, pieces[k].bytes);
+            else std::memset(pieces[k].dst, 0, pieces[k].bytes);
+        }
+    };
+    const size_t nt = std::min<size_t>({8, total / (2u << 20) + 1, std::max<size_t>(pieces.size(), 1)});
+    std::vector<std::thread> th;
+    size_t started = 1;
+    try {
+        for (; started < nt; ++started) th.emplace_back(run, started, nt);
+    } catch (const std::exception &) {
+        // no thread to be had: their pieces are moved here
+    }
+    run(0, nt);
+    for (size_t k = started; k < nt; ++k) run(k, nt);
+    for (std::thread &x : th) x.join();
+}
+
 template <typename R> int set_particles_impl(mpmw_solver *s, const mpmw_particle_arrays *a) {
     const int32_t n = a->n;
     bool back = s->prm.kinematic_hardening > 0.0;
@@ -1241,34 +1313,112 @@ template <typename R> int get_particles_impl(mpmw_solver *s, mpmw_particle_array
     HIP_TRY(hipStreamSynchronize(s->stream));
     const int32_t n = std::min(a->n, s->n);
     int rc;
-    struct { int fld; double *dst; int comp, c; } map[] = {
-        {F_X, a->pos, 3, 0}, {F_Y, a->pos, 3, 1}, {F_Z, a->pos, 3, 2},
-        {F_VX, a->vel, 3, 0}, {F_VY, a->vel, 3, 1}, {F_VZ, a->vel, 3, 2},
-        {F_S0, a->stress, 6, 0}, {F_S1, a->stress, 6, 1}, {F_S2, a->stress, 6, 2},
-        {F_S3, a->stress, 6, 3}, {F_S4, a->stress, 6, 4}, {F_S5, a->stress, 6, 5},
-        {F_EPS, a->plastic_strain, 1, 0}, {F_RATE, a->strain_rate, 1, 0},
-        {F_DMG, a->damage, 1, 0}, {F_SRES, a->residual_stress, 1, 0},
-        {F_T, a->temperature, 1, 0}, {F_M, a->mass, 1, 0}, {F_V, a->volume, 1, 0},
-        {F_DENS, a->density, 1, 0},
-        {F_A0, a->backstress, 6, 0}, {F_A1, a->backstress, 6, 1}, {F_A2, a->backstress, 6, 2},
-        {F_A3, a->backstress, 6, 3}, {F_A4, a->backstress, 6, 4}, {F_A5, a->backstress, 6, 5},
-        {F_FX, a->fext, 3, 0}, {F_FY, a->fext, 3, 1}, {F_FZ, a->fext, 3, 2},
+    // the first field of each array and its components
+    struct { int fld; void *dst; int comp; } map[] = {
+        {F_X, a->pos, 3}, {F_VX, a->vel, 3}, {F_S0, a->stress, 6}, {F_EPS, a->plastic_strain, 1},
+        {F_RATE, a->strain_rate, 1}, {F_DMG, a->damage, 1}, {F_SRES, a->residual_stress, 1},
+        {F_T, a->temperature, 1}, {F_M, a->mass, 1}, {F_V, a->volume, 1}, {F_DENS, a->density, 1},
+        {F_A0, a->backstress, 6}, {F_FX, a->fext, 3}, {F_STATUS, a->status, 1}, {F_ID, a->id, 1},
     };
-    for (auto &e : map) {
-        if (!e.dst || n == 0) continue;
-        if (!field_live(s, e.fld)) {
-            for (int64_t i = 0; i < n; ++i) e.dst[i * e.comp + e.c] = 0.0;
-            continue;
-        }
-        rc = is_pos(e.fld) ? download_field<double>(s, e.fld, e.dst, n, e.comp, e.c)
-                           : download_field<R>(s, e.fld, e.dst, n, e.comp, e.c);
-        if (rc) return rc;
+    static_assert(F_Z == F_X + 2 && F_VZ == F_VX + 2 && F_S5 == F_S0 + 5 && F_A5 == F_A0 + 5 && F_FZ == F_FX + 2,
+                  "components in order");
+    std::vector<mpmw_internal::ReadArray> out;
+    for (const auto &e : map) {
+        if (!e.dst) continue;
+        mpmw_internal::ReadArray r;
+        r.dst = e.dst;
+        r.comp = e.comp;
+        r.kind = e.fld >= kNumReal ? mpmw_internal::kReadI32
+                                   : (is_pos(e.fld) || sizeof(R) == 8 ? mpmw_internal::kReadF64 : mpmw_internal::kReadF32);
+        if (!field_live(s, e.fld)) r.kind = mpmw_internal::kReadZero;
+        for (int c = 0; c < e.comp; ++c) r.src[c] = s->f[e.fld + c];
+        out.push_back(r);
     }
-    if (n > 0 && a->status) HIP_TRY(hipMemcpy(a->status, s->f[F_STATUS], sizeof(int32_t) * n, hipMemcpyDeviceToHost));
-    if (n > 0 && a->id) HIP_TRY(hipMemcpy(a->id, s->f[F_ID], sizeof(int32_t) * n, hipMemcpyDeviceToHost));
+    if ((rc = mpmw_internal::read_back(s->prm.device, s->stream, out, n))) return rc;
     a->n = n;
     return MPMW_OK;
 }
+
+}  // namespace
+
+namespace mpmw_internal {
+
+int read_back(int device, hipStream_t stream, const std::vector<ReadArray> &arrays, int64_t n) {
+    constexpr size_t kChunk = 32u << 20;
+    // the arrays cut into chunks of whole rows
+    struct Chunk {
+        ReadTable t{};
+        int np = 0;
+        size_t bytes = 0;
+        std::vector<HostMove> moves;   // src: the offset in the chunk
+    };
+    std::vector<Chunk> chunks;
+    std::vector<HostMove> zeros;
+    for (const ReadArray &a : arrays) {
+        if (!a.dst || n <= 0) continue;
+        const size_t row = a.kind == kReadI32 ? sizeof(int32_t) : sizeof(double) * (size_t)a.comp;
+        if (a.kind == kReadZero) {
+            zeros.push_back({(char *)a.dst, nullptr, row * (size_t)n});
+            continue;
+        }
+        for (int64_t i = 0; i < n;) {
+            if (chunks.empty() || chunks.back().np == kReadPieces || chunks.back().bytes + row > kChunk)
+                chunks.emplace_back();
+            Chunk &c = chunks.back();
+            const int64_t k = std::min<int64_t>(n - i, (int64_t)((kChunk - c.bytes) / row));
+            ReadPiece &p = c.t.p[c.np++];
+            for (int q = 0; q < a.comp; ++q) p.src[q] = a.src[q];
+            p.i0 = i;
+            p.at = c.bytes;
+            p.count = (int32_t)k;
+            p.comp = a.comp;
+            p.kind = a.kind;
+            p.ones = a.ones;
+            c.moves.push_back({(char *)a.dst + row * (size_t)i, (const char *)c.bytes, row * (size_t)k});
+            c.bytes += (row * (size_t)k + 255) & ~(size_t)255;
+            i += k;
+        }
+    }
+    if (chunks.empty()) {
+        move_out(zeros);
+        return MPMW_OK;
+    }
+    // a pinned area for the chunk under way and one for the chunk before it
+    size_t area = 1u << 20;
+    for (const Chunk &c : chunks) while (area < c.bytes) area *= 2;
+    const size_t areas = chunks.size() > 1 ? 2 : 1;
+    void *stage = nullptr;
+    hipEvent_t ev[2] = {nullptr, nullptr};
+    hipError_t e = pool::get(device, true, areas * area, &stage);
+    for (size_t k = 0; k < areas && e == hipSuccess; ++k) e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
+    auto out = [&](size_t k) {
+        e = hipEventSynchronize(ev[k % areas]);
+        if (e != hipSuccess) return;
+        std::vector<HostMove> m = chunks[k].moves;
+        for (HostMove &x : m) x.src = (const char *)stage + (k % areas) * area + (size_t)x.src;
+        if (k + 1 == chunks.size()) m.insert(m.end(), zeros.begin(), zeros.end());
+        move_out(m);
+    };
+    for (size_t k = 0; k < chunks.size() && e == hipSuccess; ++k) {
+        const int nb = std::min(blocks_for(chunks[k].bytes / sizeof(double) / chunks[k].np + 1), 256);
+        hipLaunchKernelGGL(k_read_back, dim3(nb, chunks[k].np), dim3(kBlock), 0, stream, chunks[k].t,
+                           (char *)stage + (k % areas) * area);
+        e = hipGetLastError();
+        if (e == hipSuccess) e = hipEventRecord(ev[k % areas], stream);
+        if (e == hipSuccess && k > 0) out(k - 1);
+    }
+    if (e == hipSuccess) out(chunks.size() - 1);
+    (void)hipStreamSynchronize(stream);
+    for (hipEvent_t x : ev)
+        if (x) (void)hipEventDestroy(x);
+    pool::put(stage);
+    if (e != hipSuccess) return fail(MPMW_E_HIP, std::string("read-back: ") + hipGetErrorString(e));
+    return MPMW_OK;
+}
+
+}  // namespace mpmw_internal
+
+namespace {
 
 // initializeParticleBox / initializeCylindricalWorkpiece lattice, host side.
 struct Lattice {
