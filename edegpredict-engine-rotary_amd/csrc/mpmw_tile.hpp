@@ -658,6 +658,107 @@ template <typename R, int N> __device__ __forceinline__ void store_window(R *dst
     }
 }
 
+// The walk of a tile's particles by workgroups whose thread t owns cell t:
+// the particle of the thread's cell in slot s.  In uniform tiles that is
+// b0 + s * kBlock + tid; in tiles whose non-empty cells hold equal counts (a
+// workpiece's boundary tiles) b0 + s * nnz + the cell's rank among them, found
+// once; otherwise the slot-major position (cells with more than s particles,
+// in key order), from a ballot and a prefix over the waves: in tiles of fewer
+// than kSlotTab slots from a table of every wave's count of cells holding more
+// than s particles, made once behind one barrier (a barrier per slot holds
+// the four waves in step, so no wave's memory latency overlaps another's
+// compute: the table made the 64-workpiece batched run 8 % faster), else
+// through a barrier per slot.  The constructor and at() are called by every
+// thread of the workgroup, at() for rising slots; the constructor holds a
+// barrier.
+struct TileSlotsShared {
+    int32_t cnt[2][kBlock / kWave];
+    int32_t red[3][kBlock / kWave];
+    int32_t tab[kBlock / kWave][kSlotTab];
+};
+
+struct TileSlots {
+    static constexpr int kWaves = kBlock / kWave;
+    TileSlotsShared &sh;
+    const int b0, cnt;   // the tile's first particle, the particles of the thread's cell
+    const int tid, lane, wv;
+    int maxc;            // the largest count of the tile's cells
+    bool uniform, semi, tab;
+    int base = 0, nnz = 0, rank_nz = 0;
+    unsigned long long lt;
+
+    __device__ __forceinline__ TileSlots(TileSlotsShared &shared, int first, int count)
+        : sh(shared), b0(first), cnt(count), tid(threadIdx.x), lane(tid % kWave), wv(tid / kWave) {
+        lt = lane ? (~0ull >> (64 - lane)) : 0ull;
+        int mx = cnt, mn = cnt, mnz = cnt > 0 ? cnt : INT32_MAX;
+#pragma unroll
+        for (int o = kWave / 2; o > 0; o >>= 1) {
+            mx = max(mx, __shfl_xor(mx, o, kWave));
+            mn = min(mn, __shfl_xor(mn, o, kWave));
+            mnz = min(mnz, __shfl_xor(mnz, o, kWave));
+        }
+        if (lane == 0) { sh.red[0][wv] = mx; sh.red[1][wv] = mn; sh.red[2][wv] = mnz; }
+        __syncthreads();
+        int minc = sh.red[1][0], minnz = sh.red[2][0];
+        maxc = sh.red[0][0];
+        for (int w = 1; w < kWaves; ++w) {
+            maxc = max(maxc, sh.red[0][w]);
+            minc = min(minc, sh.red[1][w]);
+            minnz = min(minnz, sh.red[2][w]);
+        }
+        uniform = maxc == minc;
+        semi = !uniform && minnz == maxc;
+        tab = !uniform && !semi && maxc < kSlotTab;
+        if (semi) {  // uniform over the workgroup
+            const unsigned long long m = __ballot(cnt > 0);
+            if (lane == 0) sh.cnt[0][wv] = __popcll(m);
+            __syncthreads();
+            for (int w = 0; w < kWaves; ++w) {
+                const int c = sh.cnt[0][w];
+                rank_nz += (w < wv) ? c : 0;
+                nnz += c;
+            }
+            rank_nz += __popcll(m & lt);
+        }
+        if (tab) {  // uniform over the workgroup
+            for (int sl = 0; sl <= maxc; ++sl) {
+                const unsigned long long m = __ballot(cnt > sl);
+                if (lane == 0) sh.tab[wv][sl] = __popcll(m);
+            }
+            __syncthreads();
+        }
+    }
+
+    __device__ __forceinline__ int index(int sl) {
+        if (uniform) return b0 + sl * kBlock + tid;
+        if (semi) return b0 + sl * nnz + rank_nz;
+        const unsigned long long mask = __ballot(cnt > sl);
+        if (!tab) {
+            if (lane == 0) sh.cnt[sl & 1][wv] = __popcll(mask);
+            __syncthreads();
+        }
+        int before = 0, total = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+            // (a slot past the table is past every cell's last particle)
+            const int c = tab ? sh.tab[w][min(sl, kSlotTab - 1)] : sh.cnt[sl & 1][w];
+            before += (w < wv) ? c : 0;
+            total += c;
+        }
+        const int idx = b0 + base + before + __popcll(mask & lt);
+        base += total;
+        return idx;
+    }
+
+    // the index of slot `to`, slots from `from` on not yet passed (the prefix
+    // of an uneven tile runs over every slot)
+    __device__ __forceinline__ int at(int from, int to) {
+        if (!uniform && !semi)
+            for (int s = from; s < to; ++s) (void)index(s);
+        return index(to);
+    }
+};
+
 template <typename R, bool DO_G2P, bool DO_P2G, bool HAS_BACK, bool DET>
 __device__ __forceinline__ void tile_block(const Particles<R> &P, const GridView<R> &g, const Grid<R> &G,
                                            const Material<R> &M, R dt, double dtd, double zcut, G2PFlags flags,
@@ -667,9 +768,7 @@ __device__ __forceinline__ void tile_block(const Particles<R> &P, const GridView
     constexpr int kNodeBytes = DO_G2P ? WN * (int)sizeof(vec4_t<R>) : 0;
     constexpr int kAccBytes = DO_P2G ? 8 * WN * (int)sizeof(R) : 0;
     __shared__ __align__(32) unsigned char smem[kNodeBytes + kAccBytes + 32];
-    __shared__ int32_t s_cnt[2][kBlock / kWave];
-    __shared__ int32_t s_red[3][kBlock / kWave];
-    __shared__ int32_t s_tab[kBlock / kWave][kSlotTab];   // uneven tiles: cells per wave holding more than s
+    __shared__ TileSlotsShared s_slots;
     __shared__ int32_t s_q[DO_P2G && !DET ? kExcQueue : 1];  // particles whose P2G left their home cell
     __shared__ int32_t s_qn;
     vec4_t<R> *s_node = reinterpret_cast<vec4_t<R> *>(smem);
@@ -680,7 +779,7 @@ __device__ __forceinline__ void tile_block(const Particles<R> &P, const GridView
     const bool stats = DO_G2P && !DO_P2G && flags.stats != 0;
     const int tid = threadIdx.x;
     const int t = block / parts, part0 = block - t * parts;   // the tile, this workgroup's first slot
-    const int lane = tid % kWave, wv = tid / kWave;
+    const int lane = tid % kWave;
     const int hx = tid % TX, hy = (tid / TX) % TY, hz = tid / (TX * TY);
     const int tx = t % tg.ntx, ty = (t / tg.ntx) % tg.nty, tz = t / (tg.ntx * tg.nty);
     const int wx0 = tg.ox + tx * TX, wy0 = tg.oy + ty * TY, wz0 = tg.oz + tz * TZ;
@@ -722,28 +821,8 @@ __device__ __forceinline__ void tile_block(const Particles<R> &P, const GridView
                 if (w < WN) s_node[w] = window_record<R>(wrec[r]);
             }
         }
-        // largest and smallest particle count of the tile's cells, and the
-        // smallest of its non-empty cells
-        int mx = cnt, mn = cnt, mnz = cnt > 0 ? cnt : INT32_MAX;
-#pragma unroll
-        for (int o = kWave / 2; o > 0; o >>= 1) {
-            mx = max(mx, __shfl_xor(mx, o, kWave));
-            mn = min(mn, __shfl_xor(mn, o, kWave));
-            mnz = min(mnz, __shfl_xor(mnz, o, kWave));
-        }
-        if (lane == 0) { s_red[0][wv] = mx; s_red[1][wv] = mn; s_red[2][wv] = mnz; }
-        __syncthreads();
-        int maxc = s_red[0][0], minc = s_red[1][0], minnz = s_red[2][0];
-        for (int w = 1; w < kBlock / kWave; ++w) {
-            maxc = max(maxc, s_red[0][w]);
-            minc = min(minc, s_red[1][w]);
-            minnz = min(minnz, s_red[2][w]);
-        }
-        const bool uniform = (maxc == minc);
-        // every non-empty cell holds maxc particles (a workpiece's boundary
-        // tiles): slot s of the cell of rank q among the non-empty cells is
-        // particle b0 + s * nnz + q, found once instead of per slot
-        const bool semi = !uniform && minnz == maxc;
+        TileSlots slots(s_slots, b0, cnt);   // its barrier puts the window and zeros in place
+        const int maxc = slots.maxc;
 
         // home cell: its global cell index
         const int hgx = wx0 + hx, hgy = wy0 + hy, hgz = wz0 + hz;
@@ -757,67 +836,6 @@ __device__ __forceinline__ void tile_block(const Particles<R> &P, const GridView
         }
         int my_oow = 0, my_exc = 0, my_acc = 0;
         const unsigned long long lt = lane ? (~0ull >> (64 - lane)) : 0ull;
-        int base = 0;
-        int nnz = 0, rank_nz = 0;
-        if (semi) {  // uniform over the workgroup
-            const unsigned long long m = __ballot(cnt > 0);
-            if (lane == 0) s_cnt[0][wv] = __popcll(m);
-            __syncthreads();
-            for (int w = 0; w < kBlock / kWave; ++w) {
-                const int c = s_cnt[0][w];
-                rank_nz += (w < wv) ? c : 0;
-                nnz += c;
-            }
-            rank_nz += __popcll(m & lt);
-        }
-        // Uneven tiles of fewer than kSlotTab slots: every wave's count of
-        // cells holding more than s particles, for every s, in one table
-        // behind one barrier.  (A barrier per slot holds the four waves in
-        // step, so no wave's memory latency overlaps another's compute: the
-        // table made the 64-workpiece batched run 8 % faster.)
-        const bool tab = !uniform && !semi && maxc < kSlotTab;
-        if (tab) {  // uniform over the workgroup
-            for (int sl = 0; sl <= maxc; ++sl) {
-                const unsigned long long m = __ballot(cnt > sl);
-                if (lane == 0) s_tab[wv][sl] = __popcll(m);
-            }
-            __syncthreads();
-        }
-        // Particle index of this thread's cell in slot s: uniform tiles
-        // b0 + s * kBlock + tid, tiles whose non-empty cells hold equal
-        // counts b0 + s * nnz + rank; otherwise the slot-major position
-        // (cells with more than s particles, in key order), from a ballot
-        // and a prefix over the waves (from the table, else through a
-        // barrier per slot).
-        auto slot_index = [&](int sl) -> int {
-            if (uniform) return b0 + sl * kBlock + tid;
-            if (semi) return b0 + sl * nnz + rank_nz;
-            if (tab) {
-                const unsigned long long mask = __ballot(cnt > sl);
-                int before = 0, total = 0;
-#pragma unroll
-                for (int w = 0; w < kBlock / kWave; ++w) {
-                    const int c = s_tab[w][sl];
-                    before += (w < wv) ? c : 0;
-                    total += c;
-                }
-                const int idx = b0 + base + before + __popcll(mask & lt);
-                base += total;
-                return idx;
-            }
-            const unsigned long long mask = __ballot(cnt > sl);
-            if (lane == 0) s_cnt[sl & 1][wv] = __popcll(mask);
-            __syncthreads();
-            int before = 0, total = 0;
-            for (int w = 0; w < kBlock / kWave; ++w) {
-                const int c = s_cnt[sl & 1][w];
-                before += (w < wv) ? c : 0;
-                total += c;
-            }
-            const int idx = b0 + base + before + __popcll(mask & lt);
-            base += total;
-            return idx;
-        };
         // A slot's G2P inputs are loaded one slot ahead (slot 0 in the
         // prologue), unconditionally (a branch joining two versions of them
         // would move the loaded registers, waiting for the loads on the
@@ -904,15 +922,8 @@ __device__ __forceinline__ void tile_block(const Particles<R> &P, const GridView
                 }
             }
         };
-        // the index of slot `to`, slots from `from` on not yet passed (the
-        // prefix of an uneven tile runs over every slot)
-        auto slot_at = [&](int from, int to) -> int {
-            if (!uniform && !semi)
-                for (int s = from; s < to; ++s) (void)slot_index(s);
-            return slot_index(to);
-        };
-        int i_next = slot_at(0, part0);
-        if (DO_G2P && !uniform) load_g2p_in(P, cnt > part0 ? i_next : b0, nxt);
+        int i_next = slots.at(0, part0);
+        if (DO_G2P && !slots.uniform) load_g2p_in(P, cnt > part0 ? i_next : b0, nxt);
         for (int s = part0; s < maxc; s += parts) {
             G2PIn<R> cur;
             if (DO_G2P) {
@@ -927,7 +938,7 @@ __device__ __forceinline__ void tile_block(const Particles<R> &P, const GridView
             }
             flush();
             const int i = i_next;
-            i_next = slot_at(s + 1, s + parts);
+            i_next = slots.at(s + 1, s + parts);
             if (DO_G2P) load_g2p_in(P, cnt > s + parts ? i_next : b0, nxt);
             process(cur, i, cnt > s);
         }
