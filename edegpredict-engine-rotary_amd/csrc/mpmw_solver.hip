@@ -768,28 +768,34 @@ int64_t occupied_tiles(const mpmw_solver *s) {
     return tiles(s->nx, TX) * tiles(s->ny, TY) * tiles(s->nz, TZ);
 }
 
-// Workgroups that share each tile of a launch of `tiles` occupied tiles.  A workgroup
-// walks its tile's slots (8 in a slab) one after another, each a chain of
-// loads and dependent arithmetic, so a launch of fewer workgroups than the
-// chip holds at once (256 CUs, 2 each in FP32, 1 in FP64) takes as long as
-// one tile however small it is: 27 tiles (20 thousand particles) 56 us, 64
-// (131 thousand) 63 us.  Sharing a tile costs its prologue and its window
-// once more, so tiles are shared only while the launch then still fits the
-// chip in one go: 8 ways 18 us at 27 tiles, 8 ways 34 us at 64 (the grid
-// update, reading more windows, 9 -> 12 and 25 -> 27 us).  The
-// deterministic mode keeps one workgroup per tile: its sums must not depend
-// on what else is in the launch.  So does an FP32 workpiece under a point
-// tool: such a tool has no motion of its own, the workpiece moves through the
-// grid, and the nearly empty nodes along its moving surface turn the last
-// bits of their sums into velocity and contact heat (regrouping the sums
-// moved the temperatures of a 200-step pass by up to 5e-4, against 5e-7 under
-// a wedge or drill).
+// Workgroups that share each tile of a solver.  A workgroup walks its tile's
+// slots (8 in a slab) one after another, each a chain of loads and dependent
+// arithmetic, so a launch of fewer workgroups than the chip holds at once
+// takes as long as one tile however small it is: 27 tiles (20 thousand
+// particles) 56 us, 64 (131 thousand) 63 us.  Sharing a tile costs its
+// prologue and its window once more (and the grid update reads more
+// windows), so tiles are shared only while the solver's own workgroups then
+// still have a CU each.  A whole step: 27 tiles 8 ways 71 -> 54 us, 64 tiles 4
+// ways 76 -> 60; in FP64 27 tiles 8 ways 78 -> 62, 125 tiles 2 ways 94 -> 88.
+// The rule looks at the solver alone, never at the rest of a launch: how its
+// tiles are shared groups its P2G sums, and a member of a batch has the sums
+// of the same workpiece stepped alone.  The full chip of a batch pays for
+// that (64 workpieces, 75 steps: 218 ms without sharing, 228 with; 240 with
+// a limit of two FP32 workgroups a CU, which gained nothing alone but for 129
+// to 256 tiles, 78 -> 71 us a step).
+// The deterministic mode keeps one workgroup per tile.  So does an FP32
+// workpiece under a point tool: such a tool has no motion of its own, the
+// workpiece moves through the grid, and the nearly empty nodes along its
+// moving surface turn the last bits of their sums into velocity and contact
+// heat (regrouping the sums moved the temperatures of a 200-step pass by up
+// to 5e-4, against 5e-7 under a wedge or drill).
 constexpr int kMostParts = 8;
-int tile_sharing(const mpmw_solver *s, int64_t tiles) {
+int tile_sharing(const mpmw_solver *s) {
     if (s->deterministic || (s->tool_kind == MPMW_TOOL_POINTS && !s->fp64)) return 1;
-    const int64_t resident = s->fp64 ? 256 : 512;
+    constexpr int64_t kCUs = 256;
+    const int64_t tiles = occupied_tiles(s);
     int p = 1;
-    while (p < kMostParts && tiles * p * 2 <= resident) p *= 2;
+    while (p < kMostParts && tiles * p * 2 <= kCUs) p *= 2;
     return p;
 }
 
@@ -824,7 +830,7 @@ template <typename R> int sort_launch(mpmw_solver *s) {
         hipLaunchKernelGGL(k_fill<int32_t>, dim3(1), dim3(64), 0, s->stream, S.oow, (int64_t)3, 0);
     }
     {
-        S.most_parts = tile_sharing(s, occupied_tiles(s));
+        S.most_parts = tile_sharing(s);
         const int64_t bytes = (int64_t)tg.ntiles * S.most_parts * 8 * (s->apic ? QN : WN) * (int64_t)s->rsz;
         if (bytes > s->tpart_cap) {
             const int64_t c = std::max<int64_t>(bytes, s->tpart_cap * 5 / 4);
@@ -2707,9 +2713,8 @@ int graph_step(StepStaging &st, hipStream_t stream, size_t end, std::vector<uint
     return MPMW_OK;
 }
 
-// The tile-pass work item of a solver in a launch of `tiles` occupied tiles in all
-// (block0 is set by the caller).
-template <typename R> TileWork<R> tile_work(mpmw_solver *s, double dt, double zcut, G2PFlags fl, int64_t tiles) {
+// The tile-pass work item of a solver (block0 is set by the caller).
+template <typename R> TileWork<R> tile_work(mpmw_solver *s, double dt, double zcut, G2PFlags fl) {
     TileWork<R> t;
     t.P = pview<R>(s);
     t.g = gview<R>(s);
@@ -2726,7 +2731,7 @@ template <typename R> TileWork<R> tile_work(mpmw_solver *s, double dt, double zc
     t.counters = s->sort.oow;
     t.tpart = (R *)s->tpart;
     t.block0 = 0;
-    t.parts = s->sort.pass_parts = std::min(tile_sharing(s, tiles), s->sort.most_parts);
+    t.parts = s->sort.pass_parts = std::min(tile_sharing(s), s->sort.most_parts);
     t.blocks = t.tg.ntiles * t.parts;
     return t;
 }
@@ -2775,9 +2780,6 @@ template <typename R> int step_begin_many(mpmw_solver *const *members, size_t nm
     std::vector<TileWork<R>> pw[kTileVariants];
     std::vector<int> pm;
     int pblocks[kTileVariants] = {};
-    int64_t tiles = 0;
-    for (size_t m = 0; m < nm; ++m)
-        if (live[m] && !members[m]->p2g_ready) tiles += occupied_tiles(members[m]);
     for (size_t m = 0; m < nm; ++m) {
         if (!live[m]) continue;
         mpmw_solver *s = members[m];
@@ -2794,7 +2796,7 @@ template <typename R> int step_begin_many(mpmw_solver *const *members, size_t nm
         if ((rc = zero_acc<R>(s))) return rc;
         hipLaunchKernelGGL(k_fill<int32_t>, dim3(1), dim3(64), 0, stream, s->sort.oow + 1, (int64_t)2, 0);
         const int v = p2g_variant(s);
-        TileWork<R> t = tile_work<R>(s, dts[m], sp.zcut, G2PFlags{}, tiles);
+        TileWork<R> t = tile_work<R>(s, dts[m], sp.zcut, G2PFlags{});
         s->sort.win_parts = t.parts;
         t.block0 = pblocks[v];
         pblocks[v] += t.blocks;
@@ -2915,8 +2917,6 @@ template <typename R> int step_many(mpmw_solver *const *members, size_t nm, cons
     std::vector<SumWork> sw(nr);
     std::vector<TileWork<R>> tw[kTileVariants];
     int gblocks[kGridVariants] = {}, dblocks = 0, sblocks = 0, tblocks[kTileVariants] = {};
-    int64_t tiles = 0;
-    for (int r = 0; r < nr; ++r) tiles += occupied_tiles(members[run[r]]);
     for (int r = 0; r < nr; ++r) {
         mpmw_solver *s = members[run[r]];
         const StepPlan &sp = plans[run[r]];
@@ -2953,7 +2953,7 @@ template <typename R> int step_many(mpmw_solver *const *members, size_t nm, cons
         s->cf_chunks = sw[r].chunks;
         sw[r].counters = sp.next_rebuild ? nullptr : s->sort.oow;
         const int v = tile_variant(s, sp);
-        TileWork<R> t = tile_work<R>(s, dt, sp.zcut, sp.fl, tiles);
+        TileWork<R> t = tile_work<R>(s, dt, sp.zcut, sp.fl);
         if (!sp.next_rebuild) s->sort.win_parts = t.parts;   // the grid item above reads the last P2G's windows
         t.block0 = tblocks[v];
         tblocks[v] += t.blocks;

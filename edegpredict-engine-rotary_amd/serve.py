@@ -92,9 +92,9 @@ def state_bytes(req, precision):
     nodes = (cx + 10) * (cy + 10) * (cz + 10) * 5 // 4
     tiles = (cx // 8 + 3) * (cy // 8 + 3) * (cz // 4 + 3) * 5 // 4
     window = 847 if apic else 405
-    # a small workpiece's tiles have up to 8 windows each, while its occupied tiles' fit 512 workgroups
+    # a small workpiece's tiles have up to 8 windows each, while its occupied tiles' fit 256 workgroups
     occupied, parts = -(-cx // 8) * -(-cy // 8) * -(-cz // 4), 1
-    while parts < 8 and occupied * parts * 2 <= 512:
+    while parts < 8 and occupied * parts * 2 <= 256:
         parts *= 2
     total = n * per_particle + nodes * 14 * r + tiles * parts * 8 * window * r
     if cfg["tool"][0] == "voxel":

@@ -1,11 +1,11 @@
 """Tiles shared by several workgroups (GPU).
 
-A launch of few tiles shares each tile among 2, 4 or 8 workgroups, and how
-many depends on all the tiles of the launch, so a member of a batch changes
-between steps.  Its particles must stay those of the workpiece stepped alone:
-up to the order of the P2G sums, i.e. to rounding carried through the steps
-(1e-9 normwise in FP64, 1e-5 in FP32, the parity tests' tolerances), across a
-grid rebuild and across joining and leaving.
+A workpiece of few tiles shares each tile among 2, 4 or 8 workgroups, alone and
+in a batch.  A member's particles must stay those of the workpiece stepped
+alone: up to the order of the sums that are formed with atomics, i.e. to
+rounding carried through the steps (1e-9 normwise in FP64, 1e-5 in FP32, the
+parity tests' tolerances), across a grid rebuild and across joining and
+leaving.
 """
 import pytest
 
