@@ -184,6 +184,7 @@ struct mpmw_solver {
     double bounds[6] = {0, 0, 0, 0, 0, 0};
     bool deterministic = false;
     bool uniform_mv = false;       // every particle has mass m0 and volume V0
+    bool moving = false;           // some particle was given a velocity
     double m0 = 0.0, V0 = 0.0;
 
     // sorting
@@ -784,14 +785,16 @@ int64_t occupied_tiles(const mpmw_solver *s) {
 // a limit of two FP32 workgroups a CU, which gained nothing alone but for 129
 // to 256 tiles, 78 -> 71 us a step).
 // The deterministic mode keeps one workgroup per tile.  So does an FP32
-// workpiece under a point tool: such a tool has no motion of its own, the
-// workpiece moves through the grid, and the nearly empty nodes along its
-// moving surface turn the last bits of their sums into velocity and contact
-// heat (regrouping the sums moved the temperatures of a 200-step pass by up
-// to 5e-4, against 5e-7 under a wedge or drill).
+// workpiece that moves through the grid, as one given a velocity does and one
+// under a point tool may (such a tool has no motion of its own): the nearly
+// empty nodes along a moving surface turn the last bits of their sums into
+// velocity and contact heat.  Regrouping the sums moved the temperatures of a
+// 200-step pass of a moving workpiece by up to 5e-4 under a point tool, 6e-5
+// under a wedge, 2e-5 under a drill or voxel tool; of one at rest under a tool
+// at 5 m/s by 2e-7 in 2000 steps.
 constexpr int kMostParts = 8;
 int tile_sharing(const mpmw_solver *s) {
-    if (s->deterministic || (s->tool_kind == MPMW_TOOL_POINTS && !s->fp64)) return 1;
+    if (s->deterministic || (!s->fp64 && (s->moving || s->tool_kind == MPMW_TOOL_POINTS))) return 1;
     constexpr int64_t kCUs = 256;
     const int64_t tiles = occupied_tiles(s);
     int p = 1;
@@ -1264,6 +1267,7 @@ template <typename R> int set_particles_impl(mpmw_solver *s, const mpmw_particle
     }
     s->has_back = back;
     s->has_fext = fext;
+    s->moving = std::any_of(a->vel, a->vel + 3 * (int64_t)n, [](double v) { return v != 0.0; });
     s->n = 0;
     int rc = alloc_particles(s, n);
     if (rc) return rc;
@@ -1484,6 +1488,7 @@ template <typename R> int init_slab_impl(mpmw_solver *s, uint64_t seed, int32_t 
     }
     s->has_back = s->prm.kinematic_hardening > 0.0;
     s->has_fext = false;
+    s->moving = vel[0] != 0.0 || vel[1] != 0.0 || vel[2] != 0.0;
     s->n = 0;
     int rc = alloc_particles(s, (int32_t)n);
     if (rc) return rc;
