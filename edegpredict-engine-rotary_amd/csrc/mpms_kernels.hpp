@@ -754,19 +754,24 @@ __device__ __forceinline__ void p2g_block(const Particles<R> &P, const Grid<R> &
 // 8 q + r: workgroups go to the 8 XCDs round-robin, so both jobs run on one
 // die and the second finds the tile's positions in its L2.  Window w is part
 // w % parts of tile w / parts; the mass and momentum records of the nw
-// windows come first in tpart, then the force records.
+// windows come first in tpart, then the force records.  `fold`: one
+// workgroup does both jobs of window blockIdx.x, half the workgroups
+// (p2g_folds, mpms_solver.hip).
 template <typename R>
 __global__ void __launch_bounds__(kBlock, P2GWaves<R>::value)
     k_p2g(Particles<R> P, Grid<R> g, Mat<R> M, const StepArgs *__restrict__ sap,
-          const int32_t *__restrict__ tile_start, R *__restrict__ tpart, int nw, int parts) {
+          const int32_t *__restrict__ tile_start, R *__restrict__ tpart, int nw, int parts, int fold) {
     __shared__ R s_w[(kBlock / 64) * 4 * kWN];
     __shared__ int32_t s_own[(kBlock / 64) * kTX * kTY];   // per wave: the head owning a base-node column this round
-    const int w = (int)(blockIdx.x >> 4) * 8 + (int)(blockIdx.x & 7), job = (int)(blockIdx.x >> 3) & 1;
+    const int job = (int)(blockIdx.x >> 3) & 1;
+    const int w = fold ? (int)blockIdx.x : (int)(blockIdx.x >> 4) * 8 + (int)(blockIdx.x & 7);
     if (w >= nw) return;
-    const int t = w / parts;
-    R *const dst = tpart + ((int64_t)job * nw + w) * (kWN * 4);
-    if (job == 0) p2g_block<R, 0>(P, g, M, sap, tile_start, dst, s_w, s_own, t, w - t * parts, parts);
-    else p2g_block<R, 1>(P, g, M, sap, tile_start, dst, s_w, s_own, t, w - t * parts, parts);
+    const int t = w / parts, part = w - t * parts;
+    R *const dst = tpart + (int64_t)w * (kWN * 4);
+    if (fold || job == 0) p2g_block<R, 0>(P, g, M, sap, tile_start, dst, s_w, s_own, t, part, parts);
+    if (fold) __syncthreads();   // job 0's window has been read
+    if (fold || job == 1)
+        p2g_block<R, 1>(P, g, M, sap, tile_start, dst + (int64_t)nw * (kWN * 4), s_w, s_own, t, part, parts);
 }
 
 // Adds the windows of the non-empty tiles whose window holds lattice node

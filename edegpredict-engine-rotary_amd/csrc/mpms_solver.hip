@@ -334,12 +334,24 @@ template <typename R> int stats(mpms_solver *s, double out[kStats]) {
 // long as one tile: 131 thousand particles (64 full tiles) shared 4 ways in
 // the P2G, 146 -> 58 us, and 8 ways in the G2P, 74 -> 26 us.
 // The tiles are counted as full ones, n / 2048: a box's edge tiles and its
-// margin hold few particles or none.
+// margin hold few particles or none (131 thousand particles: 64 of 252).  The
+// box's own tiles, each of which takes its windows and workgroups whether it
+// holds particles or not, limit the sharing where a few far chips stretch the
+// box (98 thousand particles and two chips in a box of 263 thousand tiles: 71
+// GB and 9.1 ms a step when each tile was shared, 13 GB and 2.9 ms now).
 int tile_sharing(const mpms_solver *s, int64_t resident) {
     const int64_t tiles = s->n / (8 * kTX * kTY * kTZ) + 1;
     int p = 1;
-    while (p < 8 && tiles * p * 2 <= resident) p *= 2;
+    while (p < 8 && tiles * p * 2 <= resident && (int64_t)s->ntiles * p * 2 <= 4 * resident) p *= 2;
     return p;
+}
+
+// Whether one workgroup does both jobs of a tile.  An empty tile's workgroup
+// costs 0.8 ns, a second one as much again; the split saves an occupied tile
+// 22 ns, and the one serial tile of a small block 65 us.  In the box above the
+// P2G takes 233 us folded, 447 split; at 33 thousand tiles both the same.
+bool p2g_folds(const mpms_solver *s) {
+    return s->p2g_parts == 1 && s->ntiles > 80000 + 28 * (s->n / (8 * kTX * kTY * kTZ) + 1);
 }
 
 // The grid fit (every kFitEvery steps): the overflow count of the last
@@ -579,9 +591,9 @@ template <typename R> int step_impl(mpms_solver *s, double dt) {
                            s->stream, (uint32_t *)g.claim, s->nn);
         hipLaunchKernelGGL(k_zero_words, dim3(1), dim3(kBlock), 0, s->stream, (uint32_t *)(s->d_counts + 1),
                            (int64_t)6);
-        const int pp = s->p2g_parts, nw = s->ntiles * pp;
-        hipLaunchKernelGGL(k_p2g<R>, dim3((unsigned)((nw + 7) / 8 * 16)), dim3(kBlock), 0, s->stream, P, g,
-                           material<R>(s), dsa, (const int32_t *)s->tile_start, (R *)s->tpart, nw, pp);
+        const int pp = s->p2g_parts, nw = s->ntiles * pp, fold = p2g_folds(s) ? 1 : 0;
+        hipLaunchKernelGGL(k_p2g<R>, dim3((unsigned)(fold ? nw : (nw + 7) / 8 * 16)), dim3(kBlock), 0, s->stream, P, g,
+                           material<R>(s), dsa, (const int32_t *)s->tile_start, (R *)s->tpart, nw, pp, fold);
         if (s->ntool > 0)
             hipLaunchKernelGGL(k_raster<R>, dim3(blocks(s->ntool)), dim3(kBlock), 0, s->stream, g,
                                (const double *)s->d_tool_xyz, s->ntool);
