@@ -474,9 +474,10 @@ __device__ __forceinline__ void apic_g2p(const Particles<R> &P, int i, const G2P
 // FP64 takes them in memory order.  Of a tile shared by `parts` workgroups
 // each takes every parts-th slot, or run of kBlock particles, and stores a
 // window of its own.  The window goes to tpart[block] (QN node records of 8
-// channels).  counters[0] counts particles that had left their tile's window
-// (G2P) or their wave's (P2G), counters[2] is set when one was scattered into
-// the node accumulators.
+// channels).  counters[0] counts particles that took device memory in place of
+// the tile's window (G2P and P2G each), counters[2] is set when one was
+// scattered into the node accumulators, counters[3] counts the queued particles
+// that the tile's window holds.
 template <typename R, bool DO_G2P, bool DO_P2G, bool HAS_BACK>
 __device__ __forceinline__ void apic_tile_block(const Particles<R> &P, const GridView<R> &g, const Grid<R> &G,
                                                 const Material<R> &M, R dt, double dtd, double zcut,
@@ -528,7 +529,7 @@ __device__ __forceinline__ void apic_tile_block(const Particles<R> &P, const Gri
             else for (int w = tid; w < 2 * QN; w += kBlock) win[w] = z;
             if (tid == 0) s_qn = 0;
         }
-        int my_oow = 0, my_acc = 0;
+        int my_oow = 0, my_acc = 0, my_queued = 0;
         auto process = [&](const G2PIn<R> &in, int i) {
             PState<R> p;
             p.status = DO_G2P ? in.status : P.status[i];
@@ -572,10 +573,10 @@ __device__ __forceinline__ void apic_tile_block(const Particles<R> &P, const Gri
                                           quad_scatter_terms(a, q, h));
                         return;
                     }
-                    ++my_oow;
                     const int at = atomicAdd(&s_qn, 1);
                     if (at < kExcQueue) {
                         s_q[at] = i;
+                        my_queued += inxy && (unsigned)lz <= (unsigned)TZ ? 1 : 0;
                         return;
                     }
                 } else {
@@ -583,9 +584,9 @@ __device__ __forceinline__ void apic_tile_block(const Particles<R> &P, const Gri
                         quad_scatter_window(reinterpret_cast<double *>(s_acc), qnode(lx, ly, lz), q, h, a);
                         return;
                     }
-                    ++my_oow;
                 }
                 my_acc = 1;
+                ++my_oow;
                 quad_scatter_global(g, G.acc, q, h, a);
             }
         };
@@ -665,8 +666,10 @@ __device__ __forceinline__ void apic_tile_block(const Particles<R> &P, const Gri
                     const R mass = P.m ? P.m[i] : P.m0, vol = P.m ? P.V[i] : P.V0;
                     const QFrac<R> q = quad_frac(g, p.x, p.y, p.z);
                     if (quad_scatter_node(g, G.acc, reinterpret_cast<R *>(sum), q.b[0] - qx0, q.b[1] - qy0,
-                                          q.b[2] - qz0, q, h, quad_inputs(p, C, mass, vol, fex, fey, fez), tid % 32))
+                                          q.b[2] - qz0, q, h, quad_inputs(p, C, mass, vol, fex, fey, fez), tid % 32)) {
                         my_acc = 1;
+                        my_oow += tid % 32 == 0;
+                    }
                 }
                 __syncthreads();  // the queued scatters are in
 #pragma unroll
@@ -683,13 +686,15 @@ __device__ __forceinline__ void apic_tile_block(const Particles<R> &P, const Gri
                 if (w < QN) { out[2 * w] = a[r]; out[2 * w + 1] = b[r]; }
             }
         }
-        int cntv = my_oow, cnta = my_acc;
+        int cntv = my_oow, cnta = my_acc, cntq = my_queued;
 #pragma unroll
         for (int o = kWave / 2; o > 0; o >>= 1) {
             cntv += __shfl_xor(cntv, o, kWave);
             cnta |= __shfl_xor(cnta, o, kWave);
+            cntq += __shfl_xor(cntq, o, kWave);
         }
         if (lane == 0 && cntv) atomicAdd(counters, cntv);
+        if (lane == 0 && cntq) atomicAdd(counters + 3, cntq);
         if (lane == 0 && cnta) atomicOr(counters + 2, 1);
     } else if (DO_P2G) {
         zero_window<R, QN>(tpart + (int64_t)block * (8 * QN), tid);

@@ -826,11 +826,11 @@ template <typename R> int sort_launch(mpmw_solver *s) {
     if ((rc = grow32(s, S.tile_start, S.tile_cap, tg.ntiles + 1))) return rc;
     if (!S.oow) {
         void *q;
-        if ((rc = dalloc(s, &q, 3 * sizeof(int32_t)))) return rc;
+        if ((rc = dalloc(s, &q, 4 * sizeof(int32_t)))) return rc;
         S.oow = (int32_t *)q;
-        HIP_TRY(pool::get(s->prm.device, true, 4 * sizeof(int32_t), (void **)&S.h_oow));
-        S.h_oow[0] = S.h_oow[1] = S.h_oow[2] = S.h_oow[3] = 0;
-        hipLaunchKernelGGL(k_fill<int32_t>, dim3(1), dim3(64), 0, s->stream, S.oow, (int64_t)3, 0);
+        HIP_TRY(pool::get(s->prm.device, true, 5 * sizeof(int32_t), (void **)&S.h_oow));
+        for (int k = 0; k < 5; ++k) S.h_oow[k] = 0;
+        hipLaunchKernelGGL(k_fill<int32_t>, dim3(1), dim3(64), 0, s->stream, S.oow, (int64_t)4, 0);
     }
     {
         S.most_parts = tile_sharing(s);
@@ -899,6 +899,8 @@ template <typename R> int rebuild_launch(mpmw_solver *s) {
     }
     SortState &S = s->sort;
     if (S.oow) HIP_TRY(hipMemcpyAsync(S.h_oow, S.oow, sizeof(int32_t), hipMemcpyDeviceToHost, s->stream));
+    if (S.oow && s->apic)
+        HIP_TRY(hipMemcpyAsync(S.h_oow + 4, S.oow + 3, sizeof(int32_t), hipMemcpyDeviceToHost, s->stream));
     return MPMW_OK;
 }
 
@@ -919,10 +921,15 @@ template <typename R> int rebuild_finish(mpmw_solver *s, bool &sorting) {
             const double d = std::fabs(o[a] - S.origin[a]);
             need = need || (s->deterministic ? d > 0.0 : d >= 0.5 * s->h);
         }
-        // particles that left their tile window since the last binning
-        need = need || (double)*S.h_oow > 0.01 * (double)s->n * (double)std::max<int64_t>(1, S.steps_since);
+        // particles that left their tile's window since the last binning, and
+        // those of the FP32 APIC pass that left their wave's (each takes 216
+        // LDS adds one by one)
+        const double left = (double)S.h_oow[0] + (s->apic ? (double)S.h_oow[4] : 0.0);
+        need = need || left > 0.01 * (double)s->n * (double)std::max<int64_t>(1, S.steps_since);
     }
     if (S.oow) hipLaunchKernelGGL(k_fill<int32_t>, dim3(1), dim3(64), 0, s->stream, S.oow, (int64_t)1, 0);
+    if (S.oow && s->apic)
+        hipLaunchKernelGGL(k_fill<int32_t>, dim3(1), dim3(64), 0, s->stream, S.oow + 3, (int64_t)1, 0);
     S.steps_since = 0;
     if (need) {
         if ((rc = sort_launch<R>(s))) return rc;

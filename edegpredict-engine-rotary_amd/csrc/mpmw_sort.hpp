@@ -67,9 +67,11 @@ struct SortState {
     int32_t tile_cap = 0;
     // device counters: [0] particle visits outside their tile window since
     // the last rebuild, [1] particles of the last deterministic P2G pass that
-    // were not in their binned cell
+    // were not in their binned cell, [2] set when the node accumulators hold
+    // some of the P2G's sums, [3] particle visits of the FP32 APIC pass outside
+    // their wave's window but inside the tile's, since the last rebuild
     int32_t *oow = nullptr;
-    int32_t *h_oow = nullptr;          // pinned: [0, 2) copy of the counters, [2, 4) the loose range
+    int32_t *h_oow = nullptr;          // pinned: [0, 2) copy of the counters, [2, 4) the loose range, [4] counter 3
     int32_t loose_begin = 0, loose_end = 0;   // particles binned as loose (host copy)
     mpmw::ScratchBuf temp, temp2;
     double origin[3] = {0, 0, 0};      // grid origin the particles were binned on

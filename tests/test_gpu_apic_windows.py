@@ -61,3 +61,21 @@ def test_windows_match_oracle(kind, cells, prec, tol):
     for k in ("pos", "vel", "temperature", "grid_mass", "grid_momentum", "grid_force"):
         bound = 1e-3 if k == "grid_force" and prec == "fp32" and n > 1 else tol
         assert errs[k] <= bound, (k, errs[k])
+
+
+def test_out_of_window_counts_device_memory_visits():
+    """A particle that left its wave's window but not its tile's is added in
+    LDS: the diagnostics count it in neither precision.  A translation by
+    0.55 cells takes 5 % of the particles out of their wave's window (too few to
+    fill a queue), a quarter of those out of the tile's; particles that the
+    rounding of a position puts on the other side may differ."""
+    cfg, d = case("up", (17, 9, 9))
+    d["vel"][:] = np.array([0.0, 0.0, 0.55]) * H / (STEPS * DT)
+    out = {}
+    for prec in ("fp64", "fp32"):
+        s = parity.build_gpu(cfg, prec, particles=d)
+        s.run(STEPS, DT)
+        out[prec] = s.diagnostics()["out_of_window"]
+        s.close()
+    print(f"\n[out of window] {out}", flush=True)
+    assert out["fp64"] > 100 and abs(out["fp32"] - out["fp64"]) <= 0.02 * out["fp64"]
