@@ -94,9 +94,17 @@ __device__ __forceinline__ void quad_gather_add(const vec4_t<R> &nd, R w, R gx, 
     s.L[6] += nd.z * gx; s.L[7] += nd.z * gy; s.L[8] += nd.z * gz;
 }
 
+// A node record as the APIC window holds it: an empty node, or one outside
+// the grid, has no velocity and keeps the NaN that marks it (a node's
+// temperature may be negative, so no number can).
+template <typename R> __device__ __forceinline__ vec4_t<R> quad_record(vec4_t<R> nd) {
+    if (!(nd.w == nd.w)) nd.x = nd.y = nd.z = R(0);
+    return nd;
+}
+
 // G2P gather over the 27 nodes from the LDS window (base node at window
-// index wb; empty nodes and nodes outside the grid as window_record writes
-// them, (0, 0, 0, -1), so that no node needs a branch) or from device memory
+// index wb; records as quad_record writes them, so that no node needs a
+// branch) or from device memory
 // (nodes outside the grid and empty nodes skipped, g2pKernel :538, with the
 // workpiece grid's emptiness test).  From the window the sums are factored:
 // a column of three nodes along z is reduced once for its value, its z
@@ -129,8 +137,9 @@ __device__ __forceinline__ void quad_gather_window(const vec4_t<R> *s_node, int 
                     b[r] = fma(q.dw[2][k], v[r], b[r]);
                     c[r] = fma(wz[k], v[r], c[r]);
                 }
-                tz = fma(q.w[2][k], rmax(nd.w, R(0)), tz);
-                wl += nd.w >= R(0) ? q.w[2][k] : R(0);
+                const bool live = nd.w == nd.w;
+                tz = fma(q.w[2][k], live ? nd.w : R(0), tz);
+                wl += live ? q.w[2][k] : R(0);
             }
             const R w = q.w[0][i] * q.w[1][j], gx = q.dw[0][i] * q.w[1][j], gy = q.w[0][i] * q.dw[1][j];
             s.temp = fma(w, tz, s.temp);
@@ -514,9 +523,10 @@ __device__ __forceinline__ void apic_tile_block(const Particles<R> &P, const Gri
                 const int i = qx0 + w % QX, j = qy0 + (w / QX) % QY, k = qz0 + w / (QX * QY);
                 vec4_t<R> nd;
                 if (i >= 0 && j >= 0 && k >= 0 && i < g.nx && j < g.ny && k < g.nz) {
-                    nd = window_record<R>(G.node[((int64_t)k * g.ny + j) * g.nx + i]);
+                    nd = quad_record<R>(G.node[((int64_t)k * g.ny + j) * g.nx + i]);
                 } else {
-                    nd = empty_record<R>();
+                    nd.x = nd.y = nd.z = R(0);
+                    nd.w = R(__builtin_nan(""));
                 }
                 s_node[qpnode<R>(w % QX, (w / QX) % QY, w / (QX * QY))] = nd;
             }

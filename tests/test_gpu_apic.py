@@ -146,3 +146,19 @@ def test_apic_refuses_deterministic():
         s.get_affine()
     s.step(cfg["dt"])
     s.close()
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-9), ("fp32", 1e-5)])
+def test_apic_carries_negative_temperatures(prec, tol):
+    """Temperatures below zero (a scale other than Kelvin): a node that holds
+    one is not taken for an empty node.  Without conduction, which limits node
+    temperatures from below."""
+    cfg = parity.small_case(steps=5, transfer="apic")
+    cfg["params"] = dict(cfg["params"], ref_temp=-50.0, thermal_conductivity=0.0)
+    _, d = parity.build_oracle(cfg)
+    rng = np.random.default_rng(3)
+    d["temperature"][:] = rng.uniform(-45.0, 10.0, len(d["temperature"]))
+    e = parity.run_from_state(cfg, prec, d, 5)["errors"]
+    print(f"\n[apic below zero {prec}] " + " ".join(f"{k}={v:.2e}" for k, v in sorted(e.items())), flush=True)
+    for k in ("pos", "vel", "temperature", "grid_tm"):
+        assert e[k] <= tol, (k, e[k])
