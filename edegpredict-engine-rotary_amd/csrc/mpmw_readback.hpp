@@ -11,23 +11,10 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
-#include <stdint.h>
 
-#include <vector>
+#include "mpmw_readback_plan.hpp"
 
 namespace mpmw_internal {
-
-enum : int32_t { kReadF32 = 0, kReadF64 = 1, kReadI32 = 2, kReadZero = 3 };
-
-// One host array of n x comp values: component c from device array src[c]
-// (float or double, widened to double; int32 as it is, comp 1), plus 1 where
-// bit c of `ones` is set; kReadZero: zeros.
-struct ReadArray {
-    void *dst = nullptr;
-    int32_t comp = 1, kind = kReadF64;
-    uint32_t ones = 0;
-    const void *src[9] = {};
-};
 
 // Fills every array that has a destination with its first n rows, after the
 // work already on `stream`.  Returns an MPMW_* status.

@@ -265,7 +265,12 @@ hipError_t get(int dev, bool host, size_t bytes, void **out) {
         }
         (void)hipGetLastError();
         e = host ? hipHostMalloc(out, c, hipHostMallocDefault) : hipMalloc(out, c);
-        if (e != hipSuccess) return e;
+        if (e != hipSuccess) {
+            // the caller has the error; the launch check after the next
+            // launch must not find it
+            (void)hipGetLastError();
+            return e;
+        }
         live_blocks[*out] = key;
         return e;
     }
@@ -1189,19 +1194,9 @@ template <typename R> int download_field(mpmw_solver *s, int fld, double *dst, i
     return MPMW_OK;
 }
 
-// A part of one array on its way out: `count` rows from row i0 on, at byte
-// `at` of the chunk.
-struct ReadPiece {
-    const void *src[9];
-    int64_t i0;
-    uint64_t at;
-    int32_t count, comp, kind;
-    uint32_t ones;
-};
-constexpr int kReadPieces = 24;
-struct ReadTable {
-    ReadPiece p[kReadPieces];
-};
+using mpmw_internal::HostMove;
+using mpmw_internal::ReadPiece;
+using mpmw_internal::ReadTable;
 
 __global__ void __launch_bounds__(kBlock) k_read_back(ReadTable t, char *out) {
     const ReadPiece &p = t.p[blockIdx.y];
@@ -1220,13 +1215,6 @@ __global__ void __launch_bounds__(kBlock) k_read_back(ReadTable t, char *out) {
         reinterpret_cast<double *>(out + p.at)[e] = v;
     }
 }
-
-// Host moves in parallel: (dst, src, bytes), src null for zeros.
-struct HostMove {
-    char *dst;
-    const char *src;
-    size_t bytes;
-};
 
 // The moves shared out in pieces of a megabyte among up to eight threads, one
 // for each two megabytes (most of the time of a move into fresh pageable
@@ -1361,59 +1349,27 @@ template <typename R> int get_particles_impl(mpmw_solver *s, mpmw_particle_array
 namespace mpmw_internal {
 
 int read_back(int device, hipStream_t stream, const std::vector<ReadArray> &arrays, int64_t n) {
-    constexpr size_t kChunk = 32u << 20;
-    // the arrays cut into chunks of whole rows
-    struct Chunk {
-        ReadTable t{};
-        int np = 0;
-        size_t bytes = 0;
-        std::vector<HostMove> moves;   // src: the offset in the chunk
-    };
-    std::vector<Chunk> chunks;
-    std::vector<HostMove> zeros;
-    for (const ReadArray &a : arrays) {
-        if (!a.dst || n <= 0) continue;
-        const size_t row = a.kind == kReadI32 ? sizeof(int32_t) : sizeof(double) * (size_t)a.comp;
-        if (a.kind == kReadZero) {
-            zeros.push_back({(char *)a.dst, nullptr, row * (size_t)n});
-            continue;
-        }
-        for (int64_t i = 0; i < n;) {
-            if (chunks.empty() || chunks.back().np == kReadPieces || chunks.back().bytes + row > kChunk)
-                chunks.emplace_back();
-            Chunk &c = chunks.back();
-            const int64_t k = std::min<int64_t>(n - i, (int64_t)((kChunk - c.bytes) / row));
-            ReadPiece &p = c.t.p[c.np++];
-            for (int q = 0; q < a.comp; ++q) p.src[q] = a.src[q];
-            p.i0 = i;
-            p.at = c.bytes;
-            p.count = (int32_t)k;
-            p.comp = a.comp;
-            p.kind = a.kind;
-            p.ones = a.ones;
-            c.moves.push_back({(char *)a.dst + row * (size_t)i, (const char *)c.bytes, row * (size_t)k});
-            c.bytes += (row * (size_t)k + 255) & ~(size_t)255;
-            i += k;
-        }
-    }
+    void *stage = nullptr;
+    hipError_t e = hipSuccess;
+    const ReadPlan p = stage_read_back(arrays, n, [&](size_t bytes) {
+        e = pool::get(device, true, bytes, &stage);
+        return e == hipSuccess;
+    });
+    if (e != hipSuccess) return fail(MPMW_E_NOMEM, std::string("read-back: no pinned memory: ") + hipGetErrorString(e));
+    const std::vector<ReadChunk> &chunks = p.chunks;
     if (chunks.empty()) {
-        move_out(zeros);
+        move_out(p.zeros);
         return MPMW_OK;
     }
-    // a pinned area for the chunk under way and one for the chunk before it
-    size_t area = 1u << 20;
-    for (const Chunk &c : chunks) while (area < c.bytes) area *= 2;
-    const size_t areas = chunks.size() > 1 ? 2 : 1;
-    void *stage = nullptr;
+    const size_t areas = p.areas, area = p.area;
     hipEvent_t ev[2] = {nullptr, nullptr};
-    hipError_t e = pool::get(device, true, areas * area, &stage);
     for (size_t k = 0; k < areas && e == hipSuccess; ++k) e = hipEventCreateWithFlags(&ev[k], hipEventDisableTiming);
     auto out = [&](size_t k) {
         e = hipEventSynchronize(ev[k % areas]);
         if (e != hipSuccess) return;
         std::vector<HostMove> m = chunks[k].moves;
         for (HostMove &x : m) x.src = (const char *)stage + (k % areas) * area + (size_t)x.src;
-        if (k + 1 == chunks.size()) m.insert(m.end(), zeros.begin(), zeros.end());
+        if (k + 1 == chunks.size()) m.insert(m.end(), p.zeros.begin(), p.zeros.end());
         move_out(m);
     };
     for (size_t k = 0; k < chunks.size() && e == hipSuccess; ++k) {
@@ -1429,7 +1385,10 @@ int read_back(int device, hipStream_t stream, const std::vector<ReadArray> &arra
     for (hipEvent_t x : ev)
         if (x) (void)hipEventDestroy(x);
     pool::put(stage);
-    if (e != hipSuccess) return fail(MPMW_E_HIP, std::string("read-back: ") + hipGetErrorString(e));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(MPMW_E_HIP, std::string("read-back: ") + hipGetErrorString(e));
+    }
     return MPMW_OK;
 }
 
