@@ -265,10 +265,10 @@ template <typename R> __device__ __forceinline__ R quad_along(R u, R c, int n) {
 // only, so that none of them touches another's column (one node after
 // another: 382 us).
 // A lane takes part once it has won its base node's place in `owner`; lanes
-// that share a base node take turns, at most eight.  Slots keep the
-// order in which the particles were made, so that a wave's particles mostly
-// sit alike in their cells: of 64, 63.98 have bases of their own after 50
-// steps of a jittered slab under a drill.
+// that share a base node take turns.  Slots keep the order in which the
+// particles were made, so that a wave's particles mostly sit alike in their
+// cells: of 64, 63.99 have bases of their own after 50 steps of a jittered slab
+// under a drill.
 template <typename R>
 __device__ __forceinline__ void quad_scatter_wave(vec4_t<R> *win, uint8_t *owner, int lz, int place, int wb,
                                                   QFrac<R> q, QScatter<R> z) {
@@ -478,11 +478,57 @@ __device__ __forceinline__ void apic_g2p(const Particles<R> &P, int i, const G2P
     }
 }
 
+// The walk of a wave over the particles of its layer of cells 64 at a time,
+// whatever cells they are of.  In memory a slot's particles follow each other
+// in cell order, so the layer's share of a slot is one run, and next() fills
+// the lanes with as many of the next runs as it takes (-1 in a lane without a
+// particle; all lanes -1 past the last run).  No barriers: the counts of all
+// the tile's cells are in the wave's registers.
+struct LayerRuns {
+    static constexpr int kWaves = kBlock / kWave;
+    int cnt[kWaves];            // particles of cell `lane` of each layer
+    const int lane, wv;
+    int slot = 0, base, off = 0;   // base: first particle of the slot; off: taken of this layer's run
+
+    __device__ __forceinline__ LayerRuns(const int32_t *cells, int first)
+        : lane(threadIdx.x % kWave), wv(threadIdx.x / kWave), base(first) {
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) cnt[w] = cells[w * kWave + lane + 1] - cells[w * kWave + lane];
+    }
+
+    __device__ __forceinline__ int next() {
+        int at = -1, filled = 0;
+        while (filled < kWave) {
+            int run = 0, before = 0, total = 0;
+#pragma unroll
+            for (int w = 0; w < kWaves; ++w) {
+                const int c = __popcll(__ballot(cnt[w] > slot));
+                if (w == wv) run = c;
+                before += w < wv ? c : 0;
+                total += c;
+            }
+            if (run == 0) break;   // no cell of the layer holds more
+            const int take = min(run - off, kWave - filled);
+            if (lane >= filled && lane < filled + take) at = base + before + off + lane - filled;
+            filled += take;
+            off += take;
+            if (off == run) {
+                base += total;
+                off = 0;
+                ++slot;
+            }
+        }
+        return at;
+    }
+};
+
 // One workgroup per tile: the APIC G2P and / or P2G.  FP32: thread t owns cell
-// t of the tile and walks that cell's particles slot by slot (TileSlots);
-// FP64 takes them in memory order.  Of a tile shared by `parts` workgroups
-// each takes every parts-th slot, or run of kBlock particles, and stores a
-// window of its own.  The window goes to tpart[block] (QN node records of 8
+// t of the tile and walks that cell's particles slot by slot (TileSlots), or, in
+// a tile whose non-empty cells hold unequal counts, a wave walks its layer's
+// particles 64 at a time (LayerRuns); FP64 takes them in memory order.
+// Of a tile shared by `parts` workgroups each takes every parts-th slot, 64
+// particles of a layer or run of kBlock particles, and stores a window of its
+// own.  The window goes to tpart[block] (QN node records of 8
 // channels).  counters[0] counts particles that took device memory in place of
 // the tile's window (G2P and P2G each), counters[2] is set when one was
 // scattered into the node accumulators, counters[3] counts the queued particles
@@ -603,17 +649,44 @@ __device__ __forceinline__ void apic_tile_block(const Particles<R> &P, const Gri
         if constexpr (kOwn) {
             // its barriers put the node records and zeros in place
             TileSlots slots(s_slots, b0, cell_start[t * kTileCells + tid + 1] - cell_start[t * kTileCells + tid]);
-            // a slot's G2P inputs are loaded one slot ahead, a slot past a
-            // cell's last particle loading particle b0, unused
+            // Slot by slot an uneven tile takes as many steps as its fullest
+            // cell holds particles, with few of the lanes in most of them.
+            // A step, us, slot by slot / 64 at a time (/ the pass of before,
+            // any 256 particles at a time with compare-and-swap adds into the
+            // tile's window): 786 thousand particles at random 336 / 249
+            // (/ 403), 197 thousand at random 155 / 114 (/ 162), 2 % of the
+            // cells with 50 particles and the others with one 684 / 223
+            // (/ 251), a third missing 195 / 176 (/ 301).  Piles of thousands
+            // in a cell share their 8 base nodes and take turns: 20 cells of
+            // 4000 33.9 ms / 4.8 (/ 3.5).  In a tile whose cells hold equal
+            // counts the slots' particles sit alike in their cells, which
+            // keeps their base nodes apart.
+            const bool runs_walk = !slots.uniform && !slots.semi;
+            LayerRuns runs(cell_start + t * kTileCells, b0);
+            int s = part0;   // slots walk: the slot of i_next
+            // the index of the thread's particle `ahead` steps on, -1 for none
+            auto next_index = [&](int ahead, int from) {
+                int at = -1;
+                if (runs_walk) {
+                    for (int k = 0; k < ahead; ++k) at = runs.next();
+                } else {
+                    at = slots.at(from, s);
+                    if (slots.cnt <= s) at = -1;
+                }
+                return at;
+            };
+            // a step's G2P inputs are loaded one step ahead, a lane without a
+            // particle loading particle b0, unused
             G2PIn<R> nxt;
-            int i_next = slots.at(0, part0);
-            if (DO_G2P) load_g2p_in(P, slots.cnt > part0 ? i_next : b0, nxt);
-            for (int s = part0; s < slots.maxc; s += parts) {
+            int i_next = next_index(part0 + 1, 0);
+            if (DO_G2P) load_g2p_in(P, i_next >= 0 ? i_next : b0, nxt);
+            while (runs_walk ? __ballot(i_next >= 0) != 0 : s < slots.maxc) {
                 const G2PIn<R> cur = nxt;
-                const int i = i_next;
-                i_next = slots.at(s + 1, s + parts);
-                if (DO_G2P) load_g2p_in(P, slots.cnt > s + parts ? i_next : b0, nxt);
-                if (slots.cnt > s) process(cur, i);
+                const int i = i_next, from = s + 1;
+                s += parts;
+                i_next = next_index(parts, from);
+                if (DO_G2P) load_g2p_in(P, i_next >= 0 ? i_next : b0, nxt);
+                if (i >= 0) process(cur, i);
             }
         } else {
             // no window is a wave's own: the particles in memory order, every

@@ -79,3 +79,25 @@ def test_out_of_window_counts_device_memory_visits():
         s.close()
     print(f"\n[out of window] {out}", flush=True)
     assert out["fp64"] > 100 and abs(out["fp32"] - out["fp64"]) <= 0.02 * out["fp64"]
+
+
+@pytest.mark.parametrize("prec,tol", [("fp64", 1e-9), ("fp32", 1e-5)])
+@pytest.mark.parametrize("kind,cells", [("spread", (9, 8, 5)), ("heap", (9, 9, 5)), ("pile", (9, 9, 5)),
+                                        ("spread", (56, 48, 20)), ("pile", (56, 48, 20))])
+def test_fused_pass_on_uneven_tiles(kind, cells, prec, tol):
+    """Two steps, so that the fused pass walks the uneven tiles too, shared and
+    (210 tiles) not; a pile is one cell of 400 (the small slab's) or 700
+    particles, more than the slot table has columns."""
+    cfg, d = case("heap" if kind == "pile" else kind, cells)
+    rng = np.random.default_rng(11)
+    if kind == "pile":
+        d["pos"][5:min(705, len(d["pos"]))] = (np.array([3.0, 2.0, 1.0]) +
+                                               rng.uniform(0.0, 1.0, (min(705, len(d["pos"])) - 5, 3))) * H
+    d["stress"][:] = 0.0
+    d["vel"][:] = rng.uniform(-1.0, 1.0, 3) + 200.0 * d["pos"][:, ::-1]
+    res = parity.run_from_state(cfg, prec, d, 2)
+    errs = res["errors"]
+    print(f"\n[uneven {kind} {cells} {prec}] " + " ".join(f"{k}={v:.1e}" for k, v in sorted(errs.items())), flush=True)
+    assert res["status_mismatch"] == 0
+    for k in ("pos", "vel", "temperature", "grid_mass", "grid_momentum"):
+        assert errs[k] <= tol, (k, errs[k])
