@@ -490,10 +490,13 @@ struct LayerRuns {
     const int lane, wv;
     int slot = 0, base, off = 0;   // base: first particle of the slot; off: taken of this layer's run
 
-    __device__ __forceinline__ LayerRuns(const int32_t *cells, int first)
+    // (`use` false: no walk, nothing is loaded)
+    __device__ __forceinline__ LayerRuns(const int32_t *cells, int first, bool use)
         : lane(threadIdx.x % kWave), wv(threadIdx.x / kWave), base(first) {
+        if (use) {
 #pragma unroll
-        for (int w = 0; w < kWaves; ++w) cnt[w] = cells[w * kWave + lane + 1] - cells[w * kWave + lane];
+            for (int w = 0; w < kWaves; ++w) cnt[w] = cells[w * kWave + lane + 1] - cells[w * kWave + lane];
+        }
     }
 
     __device__ __forceinline__ int next() {
@@ -662,31 +665,35 @@ __device__ __forceinline__ void apic_tile_block(const Particles<R> &P, const Gri
             // counts the slots' particles sit alike in their cells, which
             // keeps their base nodes apart.
             const bool runs_walk = !slots.uniform && !slots.semi;
-            LayerRuns runs(cell_start + t * kTileCells, b0);
-            int s = part0;   // slots walk: the slot of i_next
-            // the index of the thread's particle `ahead` steps on, -1 for none
-            auto next_index = [&](int ahead, int from) {
-                int at = -1;
-                if (runs_walk) {
-                    for (int k = 0; k < ahead; ++k) at = runs.next();
-                } else {
-                    at = slots.at(from, s);
-                    if (slots.cnt <= s) at = -1;
-                }
+            LayerRuns runs(cell_start + t * kTileCells, b0, runs_walk);
+            // the steps in which the thread has a particle, and the steps
+            int cnt = slots.cnt, steps = slots.maxc;
+            if (runs_walk) {
+                const int layer = cell_start[t * kTileCells + (wv + 1) * kWave] - cell_start[t * kTileCells + wv * kWave];
+                cnt = (layer + kWave - 1 - lane) / kWave;
+                steps = (layer + kWave - 1) / kWave;
+            }
+            // particle s of the thread's cell is mine + s * stride
+            const int stride = slots.uniform ? kBlock : slots.nnz;
+            const int mine = b0 + (slots.uniform ? tid : slots.rank_nz);
+            // the thread's particle in step `to`, steps from `from` on not yet passed
+            auto index = [&](int from, int to) {
+                if (!runs_walk) return mine + to * stride;
+                int at = 0;
+                for (int k = from; k <= to; ++k) at = runs.next();
                 return at;
             };
-            // a step's G2P inputs are loaded one step ahead, a lane without a
-            // particle loading particle b0, unused
+            // a step's G2P inputs are loaded one step ahead, a step past a
+            // thread's last particle loading particle b0, unused
             G2PIn<R> nxt;
-            int i_next = next_index(part0 + 1, 0);
-            if (DO_G2P) load_g2p_in(P, i_next >= 0 ? i_next : b0, nxt);
-            while (runs_walk ? __ballot(i_next >= 0) != 0 : s < slots.maxc) {
+            int i_next = index(0, part0);
+            if (DO_G2P) load_g2p_in(P, cnt > part0 ? i_next : b0, nxt);
+            for (int s = part0; s < steps; s += parts) {
                 const G2PIn<R> cur = nxt;
-                const int i = i_next, from = s + 1;
-                s += parts;
-                i_next = next_index(parts, from);
-                if (DO_G2P) load_g2p_in(P, i_next >= 0 ? i_next : b0, nxt);
-                if (i >= 0) process(cur, i);
+                const int i = i_next;
+                i_next = index(s + 1, s + parts);
+                if (DO_G2P) load_g2p_in(P, cnt > s + parts ? i_next : b0, nxt);
+                if (cnt > s) process(cur, i);
             }
         } else {
             // no window is a wave's own: the particles in memory order, every
