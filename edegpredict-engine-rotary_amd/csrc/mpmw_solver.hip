@@ -189,7 +189,8 @@ struct mpmw_solver {
 
     // sorting
     SortState sort{};
-    // deterministic mode: per-tile P2G windows (ntiles x 8 x WN of R)
+    // the P2G windows: ntiles x sort.most_parts x 8 channels x WN (APIC: QN)
+    // nodes of R, sized by sort_launch
     void *tpart = nullptr;
     int64_t tpart_cap = 0;         // bytes
 
